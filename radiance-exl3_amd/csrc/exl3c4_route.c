@@ -6,7 +6,7 @@
 #include "exl3c4.h"
 #include "exl3c4_dev.h"
 
-/* the scatter's workgroup holds a counter per (wave, expert) in LDS; the router holds a token's logits in registers */
+/* the scatter's workgroups hold an expert a thread; the router holds a token's logits in registers */
 #define SCATTER_MAX_EXPERTS 1024
 #define ROUTER_MAX_EXPERTS 1024
 /* router_topk_scatter runs as one workgroup (a wave a token) up to this many tokens */

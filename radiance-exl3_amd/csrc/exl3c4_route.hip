@@ -214,104 +214,96 @@ __global__ __launch_bounds__(256) void k_router(const void* logits, int64_t n_to
     }
 }
 
-// moe_scatter by the first SC_WAVES waves of a workgroup; wave v owns the contiguous pairs [v * seg, (v + 1) * seg).
-// Pass A counts, per wave, each expert's pairs (a lane's rank among the lanes of its 64-pair chunk with the same
-// expert comes from a readlane sweep, and the last such lane adds the chunk's count); then expert_offset is the
-// exclusive scan of the totals (each thread a run of experts, a scan across the lanes, then across the waves) and
-// each wave's count becomes its first row for that expert; pass B places the pairs in order. `ids` may be in LDS.
-// LDS: cnt[SC_WAVES][n_expert] i32 and SC_WAVES wave sums. Every thread of the workgroup calls it (barriers).
-constexpr int SC_WAVES = 8;
-__device__ __forceinline__ void rank_in_chunk(int e, int lane, int n, int& rank, bool& last) {
-    rank = 0;
-    last = true;
-    for (int q = 0; q < n; ++q) {                                // the chunk's n valid lanes
-
-        const bool same = __builtin_amdgcn_readlane(e, q) == e;
-        rank += (same && q < lane) ? 1 : 0;
-        last = last && !(same && q > lane);
-    }
-}
-
-__device__ __forceinline__ int expert_of(const int32_t* ids, int i, int hi, int64_t base, int n_expert) {
-    if (i >= hi) return -1;
-    const int64_t g = (int64_t)ids[i] - base;
+// moe_scatter over many workgroups without a workspace: each of them counts every pair's expert for itself, in LDS (the
+// ids come from L2 after the first read), apart for the pairs before its segment and for the others; the totals'
+// exclusive scan is expert_offset, and the offset plus the count before the segment is each expert's first row in it.
+// The segment is then placed SC_SEG pairs at a time: a pair's rank is the number of earlier pairs of the same expert
+// among them, counted by comparing ids held in LDS (wave w compares its 64 pairs with the 64 of quarter w / 4, those
+// before its own whole). Stable by construction: no order depends on the atomics, which only count.
+// What bounds it: a workgroup's chain -- three rounds of id loads, 40 LDS atomics a thread and two scans at 40,960
+// pairs -- so the time is nearly one workgroup's, however many run: 800 us in one workgroup of 8 waves before (its ranks
+// by readlane sweeps over every pair, twice), 14 us now, 401 -> 11 us at 20,480 pairs, 29 -> 6 at 1,280.
+constexpr int SC_THREADS = 1024, SC_SEG = 256, SC_LOADS = 16, SC_MAX_WG = 256;
+__device__ __forceinline__ int expert_of(int32_t id, int64_t base, int n_expert) {
+    const int64_t g = (int64_t)id - base;
     return (g >= 0 && g < n_expert) ? (int)g : -1;
 }
 
-__device__ void scatter_body(const int32_t* ids, int T, int64_t base, int n_expert, int32_t* sorted, int32_t* off,
-                             int32_t* count, int32_t* row_of, int* cnt, int* wsum) {
-    const int tid = threadIdx.x, lane = tid & 63, v = tid >> 6;
-    const int nthr = SC_WAVES * 64;
-    const bool act = v < SC_WAVES;
-    const int seg = (T + SC_WAVES - 1) / SC_WAVES;
-    const int lo = v * seg, hi = lo + seg < T ? lo + seg : T;
-    for (int j = tid; j < SC_WAVES * n_expert; j += blockDim.x) cnt[j] = 0;
+__global__ __launch_bounds__(SC_THREADS) void k_scatter(const int32_t* ids, uint32_t T, int64_t base, int32_t n_expert,
+                                                        uint32_t seg, int32_t* sorted, int32_t* off, int32_t* count,
+                                                        int32_t* row_of) {
+    __shared__ int hist[2 * SC_THREADS];                          // counts before the segment; from it on
+    __shared__ int wsum[SC_THREADS / 64];
+    __shared__ __attribute__((aligned(16))) int eid[SC_SEG];
+    __shared__ int rank_l[SC_SEG];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const uint32_t lo = blockIdx.x * seg, hi = T - lo < seg ? T : lo + seg;   // T < 2^31: nothing wraps
+    const int mine = tid < SC_SEG && lo + tid < hi ? ids[lo + tid] : 0;   // the first SC_SEG pairs, loaded ahead
+    hist[tid] = hist[SC_THREADS + tid] = 0;
     __syncthreads();
-    if (act)
-        for (int c0 = lo; c0 < hi; c0 += 64) {                   // pass A
-            const int e = expert_of(ids, c0 + lane, hi, base, n_expert);
-            int rank;
-            bool last;
-            rank_in_chunk(e, lane, hi - c0 < 64 ? hi - c0 : 64, rank, last);
-            if (e >= 0 && last) cnt[v * n_expert + e] += rank + 1;
-        }
-    __syncthreads();
-    const int per = (n_expert + nthr - 1) / nthr;                 // thread tid: experts [tid * per, (tid + 1) * per)
-    int mine = 0;
-    if (act)
-        for (int e = tid * per; e < (tid + 1) * per && e < n_expert; ++e)
-            for (int u = 0; u < SC_WAVES; ++u) mine += cnt[u * n_expert + e];
-    int incl = mine;                                              // inclusive scan across the wave's lanes
+    for (uint32_t i0 = 0; i0 < T; i0 += SC_THREADS * SC_LOADS) {
+        int32_t f[SC_LOADS];
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(incl, d);
-        if (lane >= d) incl += o;
+        for (int j = 0; j < SC_LOADS; ++j) {
+            const uint32_t i = i0 + SC_THREADS * j + tid;
+            f[j] = ids[i < T ? i : T - 1];
+        }
+#pragma unroll
+        for (int j = 0; j < SC_LOADS; ++j) {
+            const uint32_t i = i0 + SC_THREADS * j + tid;
+            const int e = i < T ? expert_of(f[j], base, n_expert) : -1;
+            if (e >= 0) atomicAdd(&hist[(i < lo ? 0 : SC_THREADS) + e], 1);
+        }
     }
-    if (act && lane == 63) wsum[v] = incl;
     __syncthreads();
-    int run = incl - mine;                                        // rows before this thread's first expert
-    for (int u = 0; u < v && u < SC_WAVES; ++u) run += wsum[u];
-    int live = 0;
-    for (int u = 0; u < SC_WAVES; ++u) live += wsum[u];
-    if (act)
-        for (int e = tid * per; e < (tid + 1) * per && e < n_expert; ++e) {
-            off[e] = run;
-            int tot = 0;
-            for (int u = 0; u < SC_WAVES; ++u) {                  // each wave's first row for expert e
-                const int c = cnt[u * n_expert + e];
-                cnt[u * n_expert + e] = run + tot;
-                tot += c;
-            }
-            if (count) count[e] = tot;
-            run += tot;
-        }
-    if (tid == 0) off[n_expert] = live;
+    const int tot = hist[tid] + hist[SC_THREADS + tid];           // 0 past n_expert
+    const int incl = wave_scan_incl(tot);
+    if (lane == 63) wsum[wv] = incl;
     __syncthreads();
-    if (act)
-        for (int c0 = lo; c0 < hi; c0 += 64) {                   // pass B
-            const int i = c0 + lane;
-            const int e = expert_of(ids, i, hi, base, n_expert);
-            int rank;
-            bool last;
-            rank_in_chunk(e, lane, hi - c0 < 64 ? hi - c0 : 64, rank, last);
-            if (i < hi) {
-                int pos = -1;
-                if (e >= 0) {
-                    pos = cnt[v * n_expert + e] + rank;
-                    sorted[pos] = i;
-                }
-                if (row_of) row_of[i] = pos;
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (e >= 0 && last) cnt[v * n_expert + e] += rank + 1;
+    const int pre = wave_scan_incl(lane < SC_THREADS / 64 ? wsum[lane] : 0);
+    const int ex = (wv ? __builtin_amdgcn_readlane(pre, wv - 1) : 0) + incl - tot;
+    const uint32_t live = (uint32_t)__builtin_amdgcn_readlane(pre, SC_THREADS / 64 - 1);
+    hist[tid] += ex;                                              // expert tid's first row in this segment
+    if (blockIdx.x == 0) {
+        if (tid < n_expert) {
+            off[tid] = ex;
+            if (count) count[tid] = tot;
         }
-    for (int i = live + tid; i < T; i += blockDim.x) sorted[i] = -1;
-}
-
-__global__ __launch_bounds__(512) void k_scatter(const int32_t* ids, int32_t T, int64_t base, int32_t n_expert,
-                                                 int32_t* sorted, int32_t* off, int32_t* count, int32_t* row_of) {
-    extern __shared__ int sc_lds[];
-    scatter_body(ids, T, base, n_expert, sorted, off, count, row_of, sc_lds, sc_lds + SC_WAVES * n_expert);
+        if (tid == 0) off[n_expert] = (int32_t)live;
+    }
+    for (uint32_t c0 = lo; c0 < hi; c0 += SC_SEG) {               // uniform
+        const uint32_t i = c0 + tid;
+        int e = -1;
+        if (tid < SC_SEG) {
+            if (i < hi) e = expert_of(c0 == lo ? mine : ids[i], base, n_expert);
+            eid[tid] = e;
+            rank_l[tid] = 0;
+        }
+        __syncthreads();
+        const int blk = wv & 3, part = wv >> 2;                   // SC_SEG / 64 of each
+        if (part <= blk) {
+            const int own = eid[blk * 64 + lane];
+            const int upto = part < blk ? 64 : lane;
+            int r = 0;
+#pragma unroll 4
+            for (int j = 0; j < 64; j += 4) {
+                const int4 q = *(const int4*)&eid[part * 64 + j];
+                r += (q.x == own && j < upto) + (q.y == own && j + 1 < upto) + (q.z == own && j + 2 < upto) +
+                     (q.w == own && j + 3 < upto);
+            }
+            if (r) atomicAdd(&rank_l[blk * 64 + lane], r);
+        }
+        __syncthreads();
+        int pos = -1;
+        if (e >= 0) {
+            pos = hist[e] + rank_l[tid];
+            sorted[pos] = (int32_t)i;
+        }
+        if (row_of && tid < SC_SEG && i < hi) row_of[i] = pos;
+        __syncthreads();                                          // every row read before the next pairs' counts
+        if (e >= 0) atomicAdd(&hist[e], 1);
+    }
+    for (uint32_t i = live + blockIdx.x * SC_THREADS + tid; i < T; i += gridDim.x * SC_THREADS) sorted[i] = -1;
 }
 
 // moe_scatter of the router's pairs (token t's top_k ids at t * top_k .., distinct experts, at most 32 tokens and
@@ -369,9 +361,8 @@ __global__ __launch_bounds__(1024) void k_route_scatter(const void* logits, int3
     int* ids_l = rs_lds;                                          // [16 * 64]
     int* cnt = rs_lds + 16 * 64;
     const int lane = threadIdx.x & 63, t = threadIdx.x >> 6;
-    const bool small = n_tok <= 32 && n_tok * top_k <= (int)blockDim.x && n_expert <= (int)blockDim.x;
-    if (small)                                                    // the histogram's counts, zeroed while routing
-        for (int i = threadIdx.x; i < n_expert; i += blockDim.x) cnt[i] = 0;
+    // 16 tokens of at most 64 slots and 1,024 experts at most (the entry's checks): scatter_small's bounds
+    for (int i = threadIdx.x; i < n_expert; i += blockDim.x) cnt[i] = 0;   // zeroed while routing
     if (t < n_tok) {
         const Pick p = route_token<DT, RPL>(logits, (int64_t)t * pitch, n_expert, top_k, renorm, lane, cand[t]);
         if (lane < top_k) {
@@ -381,8 +372,7 @@ __global__ __launch_bounds__(1024) void k_route_scatter(const void* logits, int3
         }
     }
     __syncthreads();
-    if (small) scatter_small(ids_l, n_tok * top_k, top_k, n_expert, sorted, off, count, row_of, cnt);
-    else scatter_body(ids_l, n_tok * top_k, 0, n_expert, sorted, off, count, row_of, cnt, cnt + SC_WAVES * n_expert);
+    scatter_small(ids_l, n_tok * top_k, top_k, n_expert, sorted, off, count, row_of, cnt);
 }
 
 // moe_gather: one thread a run of 8 columns of one token; the slots in ascending order, one f32 product and one add
@@ -480,9 +470,11 @@ extern "C" int exl3c4_dev_router(const void* logits, int32_t dtype, int64_t n_to
 
 extern "C" int exl3c4_dev_scatter(const int32_t* ids, int64_t T, int64_t base, int32_t n_expert, int32_t* sorted,
                                   int32_t* off, int32_t* count, int32_t* row_of, void* stream) {
-    const uint32_t lds = (uint32_t)((SC_WAVES * n_expert + SC_WAVES) * 4);
-    hipLaunchKernelGGL(k_scatter, dim3(1), dim3(SC_WAVES * 64), lds, (hipStream_t)stream, ids, (int32_t)T, base,
-                       n_expert, sorted, off, count, row_of);
+    // a workgroup each SC_SEG pairs, up to one a CU (a segment is then several SC_SEG); one when there is no pair
+    const int64_t segs = T > 0 ? (T + SC_SEG - 1) / SC_SEG : 1, per = (segs + SC_MAX_WG - 1) / SC_MAX_WG;
+    const unsigned wgs = (unsigned)((segs + per - 1) / per);
+    hipLaunchKernelGGL(k_scatter, dim3(wgs), dim3(SC_THREADS), 0, (hipStream_t)stream, ids, (uint32_t)T, base,
+                       n_expert, (uint32_t)(per * SC_SEG), sorted, off, count, row_of);
     return launched();
 }
 
@@ -490,8 +482,7 @@ extern "C" int exl3c4_dev_route_scatter(const void* logits, int32_t dtype, int32
                                         int64_t pitch, int32_t top_k, int32_t renorm, int32_t* ids, float* w,
                                         int32_t* sorted, int32_t* off, int32_t* count, int32_t* row_of,
                                         void* stream) {
-    const int tail = SC_WAVES * n_expert + SC_WAVES > n_expert + 17 ? SC_WAVES * n_expert + SC_WAVES : n_expert + 17;
-    const uint32_t lds = (uint32_t)((16 * 64 + tail) * 4);       // ids, then scatter_body's or scatter_small's
+    const uint32_t lds = (uint32_t)((16 * 64 + n_expert + 17) * 4);   // ids, then scatter_small's
     const hipStream_t st = (hipStream_t)stream;
     if (dtype == EXL3C4_F32)
         launch_rs_dt<EXL3C4_F32>(logits, n_tok, n_expert, pitch, top_k, renorm, ids, w, sorted, off, count, row_of, lds, st);

@@ -95,6 +95,21 @@ def test_scatter_matches_the_oracle(torch_cuda, n_tok, top_k, n_expert, base, ki
         assert np.array_equal(g, w_), name
 
 
+@pytest.mark.parametrize("n_tok,top_k,n_expert,lo,hi", [
+    (255, 1, 7, 0, 7), (256, 1, 7, 0, 7), (257, 1, 7, -2, 9), (64, 4, 3, 1, 2), (6554, 10, 512, -5, 520),
+    (13200, 10, 1024, 0, 1024), (9001, 15, 1, 0, 1)])
+def test_scatter_segments_match_the_oracle(torch_cuda, n_tok, top_k, n_expert, lo, hi):
+    """k_scatter's workgroups on both sides of one segment of 256 pairs and of one segment a workgroup (256 x 256 pairs,
+    65,536: beyond it a workgroup places several in turn), with every pair on one expert, with dropped pairs and over
+    the most experts: whole numbers, equal."""
+    import oracle
+    torch = torch_cuda
+    ids = np.random.default_rng(n_tok).integers(lo, hi, (n_tok, top_k)).astype(np.int32)
+    got, want = _scatter(torch, ids, n_expert), oracle.moe_scatter_full(ids, n_expert, 0)
+    for g, w_, name in zip(got, want, ("sorted_tok", "expert_offset", "expert_count", "row_of")):
+        assert np.array_equal(g, w_), name
+
+
 @pytest.mark.parametrize("n_tok,E,top_k", [(8, 512, 10), (16, 512, 10), (40, 512, 10), (16, 8, 4), (16, 1024, 64),
                                             (3, 1, 1), (16, 64, 64), (5, 100, 7)])
 def test_router_topk_scatter_matches_the_oracle(torch_cuda, n_tok, E, top_k):
