@@ -340,11 +340,11 @@ def run_decode_layer(args, torch, exl3c4):
 
 
 # The decode loop's VALU work, read from the gfx950 assembly of k_gd<4,mul1> (the same loop body in k_gu / k_dn): an
-# iteration of two steps -- each step a wave's 32-column strip over 64 k, 2048 weights -- issues 253 VALU instructions
-# (64 v_pk_mul_lo_u16, 64 v_mad_u32_u16, 32 v_sad_u8, 32 v_sad_hi_u8, 32 v_pk_fma_f16, 18 v_alignbit_b32, 6 v_perm_b32,
-# 5 others) and 8 MFMAs. The kernel's whole issue (its start-ups, epilogues, gather) is counted by SQ_INSTS_VALU in
+# iteration of two steps -- each step a wave's 32-column strip over 64 k, 2048 weights -- issues 237 VALU instructions
+# (64 v_mul_lo_u32, 48 v_bfe_u32, 16 v_and_b32, 32 v_sad_u8, 32 v_sad_hi_u8, 32 v_pk_fma_f16, 6 v_perm_b32, 7 others)
+# and 8 MFMAs. The kernel's whole issue (its start-ups, epilogues, gather) is counted by SQ_INSTS_VALU in
 # profiles/valu_k_gd_decode.json when that profile exists, and the line uses the count.
-VALU_PER_STEP, WEIGHTS_PER_STEP = 126.5, 2048
+VALU_PER_STEP, WEIGHTS_PER_STEP = 118.5, 2048
 # A SIMD issues one wave64 VALU instruction each 4 cycles; 1024 SIMDs at MI355X's 2.4 GHz peak engine clock.
 VALU_PEAK_GINSTR = 1024 * 2.4 / 4
 

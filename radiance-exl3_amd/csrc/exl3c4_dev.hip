@@ -18,12 +18,10 @@
 //
 // THE DECODE (codebook mul1, the path's codebook). The state of position q is the 16-bit window of the segment's
 // stream ending at bit (q + 1) K, taken from the segment's K words and the previous segment's last word (one DPP
-// row_ror:2, the previous segment of the same tile sitting two lanes down, circularly). One v_alignbit_b32 yields a
-// register whose low half is one state and (for K | 16) whose high half is another; the hash x * 0x83DCD12D mod 2^32
-// is v_pk_mul_lo_u16 (the high partial product, placed in the high half by op_sel) + v_mad_u32_u16 (op_sel picks the
-// state's half), so no state is ever masked; the byte sum lands as fp16 bits 0x6400 + s through v_sad_u8 /
-// v_sad_hi_u8 for two weights at once, and one v_pk_fma_f16 forms (1024 + s) * K_INV + K_BIAS for both with one
-// rounding each -- exactly common/exl3_decode.c:47-58.
+// row_ror:2, the previous segment of the same tile sitting two lanes down, circularly). v_bfe_u32 takes a state out of a
+// word, zero-extended, and the hash x * 0x83DCD12D mod 2^32 is one v_mul_lo_u32; the byte sum lands as fp16 bits
+// 0x6400 + s through v_sad_u8 / v_sad_hi_u8 for two weights at once, and one v_pk_fma_f16 forms
+// (1024 + s) * K_INV + K_BIAS for both with one rounding each -- exactly common/exl3_decode.c:47-58.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -206,51 +204,38 @@ __device__ __forceinline__ int owner_wave(const int32_t* off, int n_expert, int 
 // ------------------------------------------------------------------------------------------------ the decode
 
 struct Mul1Consts {
-    uint32_t kh;      // 0x83DC in the high half: v_pk_mul_lo_u16 puts x * 0x83DC there, zero in the low half
-    uint32_t cl;      // 0xD12D: the low 16 bits of the multiplier
     uint32_t c6464;   // fp16 1024.0 in both halves: the byte sums add onto it
     half2_t  kinv, kbias;
 };
 
 __device__ __forceinline__ Mul1Consts mul1_consts() {
     Mul1Consts k;
-    k.kh = 0x83DC0000u;
-    k.cl = 0x0000D12Du;
     k.c6464 = 0x64006400u;
     k.kinv = half2_t{ __builtin_bit_cast(_Float16, (uint16_t)0x1EEEu), __builtin_bit_cast(_Float16, (uint16_t)0x1EEEu) };
     k.kbias = half2_t{ __builtin_bit_cast(_Float16, (uint16_t)0xC931u), __builtin_bit_cast(_Float16, (uint16_t)0xC931u) };
     return k;
 }
 
-// Two states (in half HA of ra and half HB of rb) -> their two fp16 weights in one dword, low half from ra's. Per
-// state: h = x * 0x83DCD12D mod 2^32 = (x * 0x83DC mod 2^16) << 16 + x * 0xD12D -- v_pk_mul_lo_u16 puts the high
-// partial product in the high half over a zero low half (op_sel), v_mad_u32_u16 adds x * 0xD12D reading only the
-// state's half (op_sel), so no state is masked. Then v_sad_u8 / v_sad_hi_u8 leave 0x6400 + bytesum in each half
-// (fp16 1024 + s, exact), and one v_pk_fma_f16 forms (1024 + s) * K_INV + K_BIAS for both, one rounding each.
-// Only the two v_mad_u32_u16 are asm (their op_sel half select is not reached from ordinary code, which spends a
-// shift or a mask on it), and they rewrite registers the compiler's own v_pk_mul_lo_u16 defined: the compiler keeps
-// every register an MFMA reads in its hazard windows -- a VALU write of an MFMA source needs two wait states before
-// the MFMA reads it, and one of a source C the MFMA has read needs three -- only for instructions it emitted, so no
-// asm output may be a register first written by the asm or a value an MFMA reads.
-template <int H> __device__ __forceinline__ uint32_t mul1_hi_product(uint32_t r, uint32_t kh) {
-    const ushort2_t v = __builtin_bit_cast(ushort2_t, r);
-    return __builtin_bit_cast(uint32_t, __builtin_shufflevector(v, v, H, H) * __builtin_bit_cast(ushort2_t, kh));
-}
-
-template <int HA, int HB>
-__device__ __forceinline__ uint32_t mul1_pair(uint32_t ra, uint32_t rb, const Mul1Consts& k) {
-    uint32_t ya = mul1_hi_product<HA>(ra, k.kh), yb = mul1_hi_product<HB>(rb, k.kh);
-    asm("v_mad_u32_u16 %[ya], %[ra], %[cl], %[ya] op_sel:[%c[ha],0,0,0]\n\t"
-        "v_mad_u32_u16 %[yb], %[rb], %[cl], %[yb] op_sel:[%c[hb],0,0,0]"
-        : [ya] "+v"(ya), [yb] "+v"(yb)
-        : [ra] "v"(ra), [rb] "v"(rb), [cl] "s"(k.cl), [ha] "n"(HA), [hb] "n"(HB));
-    const uint32_t s = __builtin_amdgcn_sad_hi_u8(yb, 0u, __builtin_amdgcn_sad_u8(ya, 0u, k.c6464));
+// Two states -> their two fp16 weights in one dword, low half from xa's (mul1). h = x * 0x83DCD12D mod 2^32 is one
+// v_mul_lo_u32 of the zero-extended state: gfx950 issues it at the rate of any other four-cycle VALU instruction
+// (measured, ns an instruction a SIMD, 4 waves: v_mul_lo_u32 1.93, v_mad_u32_u16 1.86, v_pk_mul_lo_u16 1.84, v_sad_u8
+// 1.82, v_bfe_u32 1.82, v_alignbit_b32 1.84), so a state costs its extraction and one instruction instead of two 16-bit
+// partial products: at K = 4 237 VALU a two-step iteration (4096 weights a wave) against 253 with v_pk_mul_lo_u16 +
+// v_mad_u32_u16 on states left in place, at K = 3 235 against 289. A layer step, same box: 128 tokens 259 -> 249 us,
+// 2048 tokens 461 -> 441, 8 tokens with K = 3 / 6 53.9 -> 49.5. Then v_sad_u8 /
+// v_sad_hi_u8 leave 0x6400 + bytesum in each half (fp16 1024 + s, exact), and one v_pk_fma_f16 forms
+// (1024 + s) * K_INV + K_BIAS for both, one rounding each (common/exl3_decode.c:47-58).
+__device__ __forceinline__ uint32_t mul1_pair(uint32_t xa, uint32_t xb, const Mul1Consts& k) {
+    const uint32_t ha = xa * 0x83DCD12Du, hb = xb * 0x83DCD12Du;
+    const uint32_t s = __builtin_amdgcn_sad_hi_u8(hb, 0u, __builtin_amdgcn_sad_u8(ha, 0u, k.c6464));
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(half2_t, s), k.kinv, k.kbias));
 }
 
-// mcg / 3inst (common/exl3_decode.c:59-66): a 32-bit hash, (h & 0x8FFF8FFF) ^ 0x3B603B60, fp16 lo + hi rounded once.
-template <int CB, int H> __device__ __forceinline__ uint16_t lop_value(uint32_t r) {
-    uint32_t x = H ? (r >> 16) : (r & 0xFFFFu);
+// mcg / 3inst (common/exl3_decode.c:59-66): a 32-bit hash, (h & 0x8FFF8FFF) ^ 0x3B603B60 (one v_bitop3), fp16 lo + hi
+// rounded once (v_add_f16 with the high half by SDWA). Both halves of a pair in one v_pk_add_f16, behind v_bitop3
+// selects, is fewer instructions (301 against 317 a two-step iteration at K = 4) and measured slower: 613 tokens at
+// K = 3 mcg 304 us a layer against 293.5.
+template <int CB> __device__ __forceinline__ uint16_t lop_value(uint32_t x) {
     x = CB == EXL3C4_CB_MCG ? x * 0xCBAC1FEDu : x * 89226354u + 64248484u;
     x = (x & 0x8FFF8FFFu) ^ 0x3B603B60u;
     const _Float16 s = __builtin_bit_cast(_Float16, (uint16_t)(x & 0xFFFFu)) +
@@ -259,37 +244,35 @@ template <int CB, int H> __device__ __forceinline__ uint16_t lop_value(uint32_t 
 }
 
 // The window of one segment as K + 1 words from least significant: v[0] = the segment's last word .. v[K - 1] its
-// first, v[K] the previous segment's last word. The state of segment position q is window bits [K (31 - q), +16).
-template <int BITS, int Q> __device__ __forceinline__ uint32_t state_reg(const uint32_t (&v)[BITS + 1]) {
-    constexpr int sh = BITS * (31 - Q);
-    constexpr int base = (sh % 32 >= 16) ? sh - 16 : sh;
-    constexpr int wb = base / 32, rb = base % 32;
-    if constexpr (rb == 0) return v[wb];
-    else return __builtin_amdgcn_alignbit(v[wb + 1], v[wb], rb);
+// first, v[K] the previous segment's last word. The state of segment position q is window bits [K (31 - q), +16),
+// zero-extended here: out of one word with v_bfe_u32 (or v_and_b32), a state across two words out of the word made of
+// the two at 16 bits, z (one v_alignbit_b32 a word, shared by the states it holds).
+template <int BITS, int Q>
+__device__ __forceinline__ uint32_t state_of(const uint32_t (&v)[BITS + 1], const uint32_t (&z)[BITS]) {
+    constexpr int sh = BITS * (31 - Q), w = sh / 32, o = sh % 32;
+    if constexpr (o < 16) return (v[w] >> o) & 0xFFFFu;
+    else return (z[w] >> (o - 16)) & 0xFFFFu;
 }
-template <int BITS, int Q> constexpr int state_half() { return (BITS * (31 - Q)) % 32 >= 16 ? 1 : 0; }
 
 // Segment positions Q, Q + 1 (Q even) -> their dword of the B operands. Position q = 8 l + j: register
 // R = 2 (j / 4) + l / 2 (B_a, B_b: column s; B_c, B_d: column s + 8), dword 2 (l % 2) + (j % 4) / 2, half j % 2.
 template <int BITS, int CB, int Q>
-__device__ __forceinline__ void decode_pair(const uint32_t (&v)[BITS + 1], uint32_t (&B)[16], const Mul1Consts& k) {
-    const uint32_t ra = state_reg<BITS, Q>(v), rb = state_reg<BITS, Q + 1>(v);
-    constexpr int ha = state_half<BITS, Q>(), hb = state_half<BITS, Q + 1>();
+__device__ __forceinline__ void decode_pair(const uint32_t (&v)[BITS + 1], const uint32_t (&z)[BITS],
+                                            uint32_t (&B)[16], const Mul1Consts& k) {
+    const uint32_t xa = state_of<BITS, Q>(v, z), xb = state_of<BITS, Q + 1>(v, z);
     uint32_t out;
-    if constexpr (CB == EXL3C4_CB_MUL1) {
-        out = mul1_pair<ha, hb>(ra, rb, k);
-    } else {
-        out = (uint32_t)lop_value<CB, ha>(ra) | ((uint32_t)lop_value<CB, hb>(rb) << 16);
-    }
+    if constexpr (CB == EXL3C4_CB_MUL1) out = mul1_pair(xa, xb, k);
+    else out = (uint32_t)lop_value<CB>(xa) | ((uint32_t)lop_value<CB>(xb) << 16);
     constexpr int l = Q >> 3, j = Q & 7, jj = j & 3;
     constexpr int R = 2 * (j >> 2) + (l >> 1), dw = 2 * (l & 1) + (jj >> 1);
     B[R * 4 + dw] = out;
 }
 
 template <int BITS, int CB, int... P>
-__device__ __forceinline__ void decode_seg_impl(const uint32_t (&v)[BITS + 1], uint32_t (&B)[16], const Mul1Consts& k,
+__device__ __forceinline__ void decode_seg_impl(const uint32_t (&v)[BITS + 1], const uint32_t (&z)[BITS],
+                                                uint32_t (&B)[16], const Mul1Consts& k,
                                                 std::integer_sequence<int, P...>) {
-    (decode_pair<BITS, CB, 2 * P>(v, B, k), ...);
+    (decode_pair<BITS, CB, 2 * P>(v, z, B, k), ...);
 }
 
 // A lane's segment as its decode window (decode_pair's v): the K words reversed, then the previous segment of the same
@@ -306,7 +289,10 @@ template <int BITS, int CB>
 __device__ __forceinline__ void decode_segment(const uint32_t (&d)[BITS], uint32_t (&B)[16], const Mul1Consts& k) {
     uint32_t v[BITS + 1];
     segment_window<BITS>(d, v);
-    decode_seg_impl<BITS, CB>(v, B, k, std::make_integer_sequence<int, 16>{});
+    uint32_t z[BITS];
+#pragma unroll
+    for (int w = 0; w < BITS; ++w) z[w] = __builtin_amdgcn_alignbit(v[w + 1], v[w], 16);
+    decode_seg_impl<BITS, CB>(v, z, B, k, std::make_integer_sequence<int, 16>{});
 }
 
 // A lane's K words of one block: K u32 at p (4-byte aligned).
