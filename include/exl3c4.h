@@ -132,7 +132,9 @@ int exl3c4_launch(const Exl3c4Op* op, void* scratch, int64_t scratch_bytes, void
  * scratch before every launch (one more dispatch). exl3c4_launch_ctr takes them from `ctr` instead: a device block of
  * at least exl3c4_ctr_bytes, 256-B aligned, that the caller zeroed once (hipMemset) and keeps -- the reference's
  * counter pool, which its row instance's init allocates and zeroes and whose blocks the fused launch leaves zero
- * (kernels/exl3r4d/launch.c:311-324; the fused launch's `ctr` argument, launch.c:464-466). The block's first int32 is
+ * (kernels/exl3r4d/launch.c:311-324; the fused launch's `ctr` argument, launch.c:464-466). Given such a block, a decode
+ * launch of at least four experts a token (top_k >= 4) runs as the single kernel below EXL3C4_GD_FUSE_MIN_T rows too,
+ * with the same bits. The block's first int32 is
  * the status word exl3c4_scratch_status describes (0: good); after a launch that left it nonzero, zero the block again.
  * Two launches that may overlap (two streams) need two blocks; launches that share one are ordered on one stream. A
  * launch that does not run that kernel does not read ctr: exl3c4_launch_ctr is then exl3c4_launch. */

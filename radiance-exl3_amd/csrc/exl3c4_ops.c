@@ -66,9 +66,16 @@ static int64_t chunk_bound(int64_t T, int64_t n_expert, int ch) {
 #ifndef GU_LDS_BUDGET
 #define GU_LDS_BUDGET (20 * 1024)
 #endif
-static int ksplit_for(int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max, int ch) {
+/* Below GD_FUSE_ROWS sorted rows of two experts a token or more, at most GU_UNITS_FEW units: there every unit is
+ * resident at once either way, and a split more only adds its start-up, its stores and its count. Measured (512 experts,
+ * 2048 / 512, K = 4, the whole step in us, limits 4096 / 2100 / 1400 / 700 with gate_up_down as one kernel): 1 token
+ * 28.3 / 26.9 / 26.7 / 25.6, 2 tokens 32.3 / 28.9 / 29.3 / 29.4, hidden 2560 and 1 token 36.2 / 32.0 / 31.7 / 33.5; as
+ * three kernels, 4096 / 1400: 2 tokens 37.9 / 35.0, 8 tokens of top-2 over 8 experts 29.7 / 28.0. One expert a token
+ * (top_k 1) may mean one live expert, whose few units need the splits: it keeps GU_UNITS. */
+#define GU_UNITS_FEW 1024
+static int ksplit_for(int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max, int ch, int64_t units) {
     int s = 1;
-    while (s < 16 && 2 * s <= nb_min && chunks * n_grp * 2 * s <= GU_UNITS) s *= 2;
+    while (s < 16 && 2 * s <= nb_min && chunks * n_grp * 2 * s <= units) s *= 2;
     while (s < 16 && 2 * s <= nb_max && (int64_t)ch * (((nb_max + s - 1) / s) * 128 + 8) * 2 > GU_LDS_BUDGET) s *= 2;
     return s;
 }
@@ -111,6 +118,15 @@ static int prefill_path(const Exl3c4Op* o, int64_t T) {
 #ifndef GD_FUSE_ROWS
 #define GD_FUSE_ROWS EXL3C4_GD_FUSE_MIN_T
 #endif
+
+/* With a counter block from the caller (exl3c4_launch_ctr, exl3c4_launch_gather), also below GD_FUSE_ROWS where a token
+ * has at least GD_FEW_TOP_K experts: they are distinct, so at least that many chunks of at most M rows are live and the
+ * kernel's chain a row runs over several of them at once (a single expert's 16 rows, measured, took 66 us there against
+ * 31 as three kernels). Without a block the counters' fill would be a dispatch of its own, and the three kernels stay. The
+ * step in us as three kernels / as one (512 experts, top-10, K = 4, the gather inside): 1 token 31.2 / 26.1, 2 tokens
+ * 35.0 / 29.3, 3 tokens 37.7 / 31.6; top-4 of 16 experts, 7 tokens 30.7 / 29.7; top-2 of 8 experts, 8 tokens 28.0 /
+ * 29.2 (so not below four). */
+#define GD_FEW_TOP_K 4
 
 /* Below that, from GEPI_ROWS rows, gate_up_down forms h once a (row, 128-block) with gate_up's epilogue kernel (a wave
  * each, all in parallel) and down stages it as given; with fewer, down's workgroups form their chunk's h while staging
@@ -172,7 +188,8 @@ static void carve(const Exl3c4Op* o, int64_t T, Carve* k) {
         }
         int s = 1;
         if (!k->pf) {   /* split-K from T, M and the geometry: ksplit_for */
-            s = ksplit_for(chunk_bound(T, o->n_expert, k->chunk), rc / 128, nb_min, nb_max, k->chunk);
+            s = ksplit_for(chunk_bound(T, o->n_expert, k->chunk), rc / 128, nb_min, nb_max, k->chunk,
+                           T < GD_FUSE_ROWS && o->top_k >= 2 ? GU_UNITS_FEW : GU_UNITS);
             k->gu_lds_pitch = (int)(((nb_max + s - 1) / s) * 128 + 8);
         }
         k->split_gu = s;
@@ -513,6 +530,13 @@ static int launch_gd1(const Exl3c4Op* o, const Carve* k, char* s, void* stream, 
     return exl3c4_dev_gd(&g, stream, EV(EXL3C4_K_GATE_UP_DOWN));
 }
 
+/* Whether a launch given the counter block `ctr` runs gate_up_down's single kernel below GD_FUSE_ROWS rows: a block too
+ * small for it (need bytes) leaves the launch as it is without one. */
+static int gd_few(const Exl3c4Op* o, const Carve* k, const void* ctr, int64_t ctr_bytes, int64_t need) {
+    return k->h_gepi && gd_pair(o) && o->T > 0 && o->top_k >= GD_FEW_TOP_K && ctr && ctr_bytes >= need &&
+           (uintptr_t)ctr % 256 == 0;
+}
+
 /* The kernels a launch runs (for exl3c4_launch_timed). */
 static int runs_kernel(const Exl3c4Op* o, const Carve* k, int kernel) {
     const int op = o->op;
@@ -537,7 +561,7 @@ static int runs_kernel(const Exl3c4Op* o, const Carve* k, int kernel) {
  *   gate_up       its GEMM (input rotation staged inside), then its epilogue
  *   down          its GEMM, whose workgroups stage (and rotate) their rows and finish their output blocks
  *   gate_up_down  gate_up's GEMM, then down's, whose workgroups build h from gate_up's partial sums; from
- *                 GD_FUSE_MIN_T rows both GEMMs in one kernel (launch_gd1)
+ *                 GD_FUSE_MIN_T rows (or fewer, gd_few) both GEMMs in one kernel (launch_gd1)
  * Prefill (launch_prefill) plans 64-row chunks of one expert first and runs one GEMM kernel a projection. */
 static int launch_impl(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream, const Ctx* t) {
     int rc;
@@ -557,7 +581,7 @@ static int launch_impl(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, 
     }
 
     if (k.pf) return launch_prefill(o, &k, s, stream, t);
-    if (k.gd1) return launch_gd1(o, &k, s, stream, t);
+    if (k.gd1 || t->ctr) return launch_gd1(o, &k, s, stream, t);
 
     if (op == EXL3C4_GATE_UP || op == EXL3C4_GU_DN) {
         Exl3c4Launch a;
@@ -638,7 +662,8 @@ int exl3c4_launch_inst(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, 
     carve(o, o->T, &k);
     if (k.gd1 && ctr && (ctr_bytes < (o->T + 1) * EXL3C4_SYNC_STRIDE * 4 || (uintptr_t)ctr % 256))
         return EXL3C4_E_SCRATCH;
-    const Ctx t = { -1, NULL, NULL, 0, k.gd1 ? (int32_t*)ctr : NULL, NULL, fail };
+    const int one = k.gd1 || gd_few(o, &k, ctr, ctr_bytes, (o->T + 1) * EXL3C4_SYNC_STRIDE * 4);
+    const Ctx t = { -1, NULL, NULL, 0, one ? (int32_t*)ctr : NULL, NULL, fail };
     return launch_impl(o, scratch, scratch_bytes, stream, &t);
 }
 
@@ -660,15 +685,16 @@ int exl3c4_launch_gather(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes
         return EXL3C4_E_ALIGN;
     Carve k;
     carve(o, o->T, &k);
-    const int fuse = k.gd1 && ctr && o->y_cols / 128 <= EXL3C4_SYNC_STRIDE;
-    if (fuse && (ctr_bytes < (o->T + 1 + o->M) * EXL3C4_SYNC_STRIDE * 4 || (uintptr_t)ctr % 256))
-        return EXL3C4_E_SCRATCH;
-    if (k.gd1 && ctr && !fuse && (ctr_bytes < (o->T + 1) * EXL3C4_SYNC_STRIDE * 4 || (uintptr_t)ctr % 256))
-        return EXL3C4_E_SCRATCH;
+    const int64_t rows_ctr = (o->T + 1) * EXL3C4_SYNC_STRIDE * 4, all_ctr = rows_ctr + o->M * EXL3C4_SYNC_STRIDE * 4;
+    const int fuse = (k.gd1 ? ctr != NULL : gd_few(o, &k, ctr, ctr_bytes, all_ctr)) &&
+                     o->y_cols / 128 <= EXL3C4_SYNC_STRIDE;
+    if (fuse && (ctr_bytes < all_ctr || (uintptr_t)ctr % 256)) return EXL3C4_E_SCRATCH;
+    if (k.gd1 && ctr && !fuse && (ctr_bytes < rows_ctr || (uintptr_t)ctr % 256)) return EXL3C4_E_SCRATCH;
     const Gather gx = { expert_w, row_of, out, out_pitch };
     const Ctx tf = { -1, NULL, NULL, 0, (int32_t*)ctr, &gx, NULL };
     if (fuse) return launch_impl(o, scratch, scratch_bytes, stream, &tf);
-    const Ctx t = { -1, NULL, NULL, 0, k.gd1 ? (int32_t*)ctr : NULL, NULL, NULL };
+    const int one = k.gd1 || gd_few(o, &k, ctr, ctr_bytes, rows_ctr);
+    const Ctx t = { -1, NULL, NULL, 0, one ? (int32_t*)ctr : NULL, NULL, NULL };
     if ((rc = launch_impl(o, scratch, scratch_bytes, stream, &t)) != EXL3C4_OK) return rc;
     return exl3c4_moe_gather(o->y, EXL3C4_BF16, o->y_pitch, expert_w, row_of, o->M, o->top_k, o->y_cols, out,
                              out_pitch, stream);

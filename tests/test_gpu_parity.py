@@ -418,6 +418,31 @@ def test_launch_gather_gives_the_bits_of_the_launch_and_the_gather(torch_cuda, s
         assert np.array_equal(outs[0], oracle.moe_gather(want_y, True, w, row_of, nt, top_k))
 
 
+@pytest.mark.parametrize("n_tok,top_k,n_expert,bits,dn_bits,cb", [
+    (1, 4, 4, 4, 4, "mul1"), (1, 10, 40, 3, 6, "mul1"), (3, 10, 24, 5, 5, "mcg"), (7, 4, 6, 8, 8, "3inst"),
+    (1, 31, 48, 2, 2, "mul1")])
+def test_few_rows_with_a_counter_block_run_as_one_kernel(torch_cuda, n_tok, top_k, n_expert, bits, dn_bits, cb):
+    """gate_up_down of 4 to 31 rows, four experts a token or more: with a zeroed counter block the single kernel gives the
+    bits of the launch without one and leaves the block zero; a block too small for it (its bytes anything) is not read,
+    and the launch runs as without one."""
+    import exl3c4 as ex
+    torch = torch_cuda
+    case = Case(seed=600 + n_tok + top_k, n_tok=n_tok, top_k=top_k, n_expert=n_expert, geoms=[(512, 256)], bits=bits,
+                cb=cb, dn_bits=dn_bits)
+    dev = Dev(case)
+    want = dev.gate_up_down()
+    N = max(d["rows"] for d in dev.tabs["dn"])
+    for small in (False, True):
+        y = dev.out(N, fill=0x1234)
+        o = dev.gd_op(y)
+        ctr = dev.guard((case.T + 1) * 256 - (256 if small else 0), fill=0x5A if small else 0)
+        print(f"T {case.T} K {bits}/{dn_bits} {cb} small block {small}", flush=True)
+        assert ex.launch_ctr(o, dev.scratch(o), ctr.view) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(y.cpu().numpy().view(np.uint16), want)
+        assert bool((ctr.view == (0x5A if small else 0)).all()) and ctr.ok()
+
+
 def test_launch_gather_with_rows_past_t_leaves_the_counter_block_good(torch_cuda):
     """row_of entries past T -- the scatter's rows of 80 pairs, the op launched over its first 70 -- name no row of
     this launch: the fused gather counts a token's slots by the same predicate (0 <= row < T) as it sums them and as
