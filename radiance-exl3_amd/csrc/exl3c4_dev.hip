@@ -1891,47 +1891,46 @@ template <int NW> __device__ __forceinline__ void zero_dead_rows(const Exl3c4Lau
     }
 }
 
-// The staged input of one 64-k step of a chunk of R = 16 NT rows: R rows x 4 groups of 16 halves, a group two 16-byte
-// loads, spread over 256 threads (H = ceil(R / 64) groups a thread; a slot past the R x 4 groups reloads the last one,
+// The staged input of KS 64-k steps of a chunk of R = 16 NT rows: R rows x 4 KS groups of 16 halves, a group two 16-byte
+// loads, spread over 256 threads (H groups a thread; a slot past the last group reloads it,
 // so that the loads stay unconditional and their waits exact). Rows past the chunk load a copy of its last row. A
-// slot's address is the step's base (wave-uniform: scalar registers) plus the slot's byte offset, fixed for the chunk
+// slot's address is the stage's base (wave-uniform: scalar registers) plus the slot's byte offset, fixed for the chunk
 // and held in a register (32 bits: 2 q pitch + 48 < 2^32 for the q < 96 rows of a chunk, which the host's choice of
 // the prefill path keeps), so the steps' loads take no address arithmetic. The groups land in LDS in row order, k in
 // order: pf_step pairs the decoded B registers to match.
-template <int NT> struct StageRegs {
-    static constexpr int H = (NT + 3) / 4;                        // slots a thread
+template <int NT, int KS> struct StageRegs {
+    static constexpr int G = 64 * NT * KS;                        // groups a stage
+    static constexpr int H = (G + 255) / 256;                     // slots a thread
     u32x4_t v[2 * H];
-    uint32_t off[H];                                              // each slot's byte offset from the step's base
+    uint32_t off[H];                                              // each slot's byte offset from the stage's base
 };
-template <int NT>
-__device__ __forceinline__ void stage_init(int64_t pitch, int nrows, StageRegs<NT>& r, int tid) {
-    constexpr int G = 64 * NT;                                    // groups a step
+template <int NT, int KS>
+__device__ __forceinline__ void stage_init(int64_t pitch, int nrows, StageRegs<NT, KS>& r, int tid) {
 #pragma unroll
-    for (int h = 0; h < StageRegs<NT>::H; ++h) {
-        const int g = min(tid + 256 * h, G - 1);
-        const uint32_t q = (uint32_t)min(g >> 2, nrows - 1), grp = (uint32_t)(g & 3);
+    for (int h = 0; h < StageRegs<NT, KS>::H; ++h) {
+        const int g = min(tid + 256 * h, StageRegs<NT, KS>::G - 1);
+        const uint32_t q = (uint32_t)min(g / (4 * KS), nrows - 1), grp = (uint32_t)(g & (4 * KS - 1));
         r.off[h] = (q * (uint32_t)pitch + grp * 16u) * 2u;
     }
 }
-// base: the step's first staged column of the chunk's first row, wave-uniform
-template <int NT> __device__ __forceinline__ void stage_load(const uint16_t* base, StageRegs<NT>& r) {
+// base: the stage's first staged column of the chunk's first row, wave-uniform
+template <int NT, int KS> __device__ __forceinline__ void stage_load(const uint16_t* base, StageRegs<NT, KS>& r) {
 #pragma unroll
-    for (int h = 0; h < StageRegs<NT>::H; ++h) {
+    for (int h = 0; h < StageRegs<NT, KS>::H; ++h) {
         const __attribute__((address_space(1))) u32x4_t* p = (const __attribute__((address_space(1))) u32x4_t*)
             ((const __attribute__((address_space(1))) char*)base + (uint64_t)r.off[h]);
         r.v[2 * h] = p[0];
         r.v[2 * h + 1] = p[1];
     }
 }
-// ... and its store into a step buffer [R][kp]
-template <int NT>
-__device__ __forceinline__ void stage_store(uint16_t* A, int kp, const StageRegs<NT>& r, int tid) {
-    constexpr int G = 64 * NT;
+// ... and its store into a stage buffer [rows][kp]
+template <int NT, int KS>
+__device__ __forceinline__ void stage_store(uint16_t* A, int kp, const StageRegs<NT, KS>& r, int tid) {
 #pragma unroll
-    for (int h = 0; h < StageRegs<NT>::H; ++h) {
+    for (int h = 0; h < StageRegs<NT, KS>::H; ++h) {
         const int g = tid + 256 * h;
-        if (g >= G) break;                                        // uniform in a wave (G is a multiple of 64)
-        const int q = g >> 2, grp = g & 3;
+        if (g >= StageRegs<NT, KS>::G) break;                     // uniform in a wave (G is a multiple of 64)
+        const int q = g / (4 * KS), grp = g & (4 * KS - 1);
         u32x4_t* d = (u32x4_t*)(A + q * kp + grp * 16);
         d[0] = r.v[2 * h];
         d[1] = r.v[2 * h + 1];
@@ -2038,56 +2037,76 @@ __device__ __forceinline__ void pf_step(const uint16_t* Ab, int kp, const uint32
 }
 
 // The prefill GEMM of one chunk (<= EXL3C4_PF_ROWS rows of one expert) against the strips of one workgroup, all of k:
-// the input streams through two LDS step buffers (64 k each, a half at a time), the next step's loads in flight while
+// the input streams through two LDS stage buffers (KS 64-k steps each, a half at a time), the next stage's loads in flight while
 // this one is multiplied; each wave decodes its strip's step once and runs it against every row tile (pf_step). NH = 1:
 // 4 waves, one staged input (columns col_off + k). NH = 2: 8 waves, two staged inputs (columns k and half_off + k),
 // thread t staging half t / 256 and wave w reading half w / 4. NT: the chunk's 16-row tiles (ceil(nrows / 16)), a
 // template argument so that the loop holds no branch on it and stages only the rows it has. Accumulations:
 // acc[row tile][strip half]. The weight: entry jx of the codes table (codes, codes_s) of k = KC columns.
-constexpr int PF_KP = EXL3C4_KSTEP + 8;                           // a staged row, padded: 16 rows hit 16 bank groups
-template <int BITS, int CB, int NH, int NT>
+//
+// KS: 64-k steps a stage. A stage costs a barrier, at which the workgroup's waves meet, so a chunk of few row tiles --
+// whose steps are little more than the decode -- takes as many steps a stage as the buffers of a seven-tile step hold:
+// four for one tile (two where k is an odd number of 128-blocks), two for two or three, one beyond. Measured against one
+// step a stage throughout (the layer step, us): 128 tokens 250 -> 234, 613 tokens with a Zipf popularity 291 -> 277,
+// 2048 Zipf 446 -> 438, 2560 / 640 at 128 tokens 364 -> 343.
+template <int KS> constexpr int pf_kp() { return KS * EXL3C4_KSTEP + 8; }   // a staged row, padded: 16 rows hit 16 bank groups
+constexpr int PF_BUF = EXL3C4_PF_ROWS * pf_kp<1>();              // halves a stage buffer of one input holds
+template <int BITS, int CB, int NH, int NT, int KS>
 __device__ __forceinline__ void pf_gemm_nt(const void* codes, int32_t codes_s, int KC, int64_t jx, int strip,
                                         const uint16_t* src, int64_t pitch, int row0, int nrows, int col_off,
                                         int half_off, uint16_t* lds, float4_t (&acc)[PF_NT][2]) {
+    static_assert(16 * NT * pf_kp<KS>() <= PF_BUF, "a stage fits its buffer");
     const int lane = threadIdx.x & 63;
-    const int nb = KC / 128, ksteps = KC / EXL3C4_KSTEP;
-    constexpr int kp = PF_KP;
+    const int nst = KC / (EXL3C4_KSTEP * KS), ksteps = KC / EXL3C4_KSTEP;
+    constexpr int kp = pf_kp<KS>();
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t][0] = acc[t][1] = float4_t{ 0.f, 0.f, 0.f, 0.f };   // the chunk's tiles only
     const int tid = (int)threadIdx.x & 255;
     const int sh = NH == 2 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;   // staged and read half
     const uint16_t* sbase = src + (int64_t)row0 * pitch + col_off + sh * half_off;   // wave-uniform
-    auto bufp = [&](int b, int h) { return lds + (b * NH + h) * EXL3C4_PF_ROWS * kp; };
+    auto bufp = [&](int b, int h) { return lds + (b * NH + h) * PF_BUF; };
     const gu32p rec = (gu32p)tab_entry(codes, codes_s, jx) + (int64_t)strip * ksteps * 64 * BITS + lane * BITS;
     // the codes of the steps ahead: dA even steps, dB odd; each refill 2 steps ahead of the step it serves (clamped:
     // past the stream a harmless reload of the last step, unconditional so that the waits count exactly)
     uint32_t dA[BITS], dB[BITS];
     load_words<BITS>(rec, dA);
     load_words<BITS>(rec + 64 * BITS, dB);
-    StageRegs<NT> r;
-    stage_init<NT>(pitch, nrows, r, tid);
-    stage_load<NT>(sbase, r);
+    StageRegs<NT, KS> r;
+    stage_init(pitch, nrows, r, tid);
+    stage_load(sbase, r);
     const Mul1Consts k = mul1_consts();
-    stage_store<NT>(bufp(0, sh), kp, r, tid);
+    stage_store(bufp(0, sh), kp, r, tid);
     __syncthreads();
     const int rr = lane & 15, g = lane >> 4;
-    int kb = 0;
-    do {                                                          // nb >= 1: the launch checks refuse k of 0
+    constexpr int U = KS > 2 ? KS : 2;                            // steps an iteration: two stages of one step, or a stage
+    int ks0 = 0, cur = 0;
+    do {                                                          // k >= 128: the launch checks refuse k of 0
+        // the next stage's loads, or at the last a harmless reload of it: unconditional, like the codes' refills
+        if (KS > 1) stage_load(sbase + min(ks0 / KS + 1, nst - 1) * (KS * EXL3C4_KSTEP), r);
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {                          // step ks = 2 kb + s2 sits in buffer s2
-            const int ks = 2 * kb + s2;
-            // the next step, or at the last a harmless reload of it: unconditional, like the codes' refills
-            stage_load<NT>(sbase + min(ks + 1, ksteps - 1) * EXL3C4_KSTEP, r);
+        for (int s = 0; s < U; ++s) {
+            const int ks = ks0 + s;
+            if (KS == 1) stage_load(sbase + min(ks + 1, nst - 1) * EXL3C4_KSTEP, r);
             uint32_t B[16];
-            decode_segment<BITS, CB>(s2 ? dB : dA, B, k);
+            decode_segment<BITS, CB>((s & 1) ? dB : dA, B, k);
             const int nx = min(ks + 2, ksteps - 1);
-            if (s2 == 0) load_words<BITS>(rec + (int64_t)nx * 64 * BITS, dA);
+            if ((s & 1) == 0) load_words<BITS>(rec + (int64_t)nx * 64 * BITS, dA);
             else load_words<BITS>(rec + (int64_t)nx * 64 * BITS, dB);
-            pf_step<BITS, CB, NT>(bufp(s2, sh) + rr * kp + 16 * g, kp, B, acc);
-            if (ks + 1 < ksteps) stage_store<NT>(bufp(s2 ^ 1, sh), kp, r, tid);
+            // step ks sits in buffer ks % 2 (KS 1), or at its place in the stage's buffer
+            const uint16_t* A = KS == 1 ? bufp(s & 1, sh) : bufp(cur, sh) + s * EXL3C4_KSTEP;
+            pf_step<BITS, CB, NT>(A + rr * kp + 16 * g, kp, B, acc);
+            if (KS == 1) {
+                if (ks + 1 < ksteps) stage_store(bufp((s & 1) ^ 1, sh), kp, r, tid);
+                __syncthreads();
+            }
+        }
+        ks0 += U;
+        if (KS > 1) {
+            cur ^= 1;
+            if (ks0 < ksteps) stage_store(bufp(cur, sh), kp, r, tid);
             __syncthreads();
         }
-    } while (++kb < nb);
+    } while (ks0 < ksteps);
 }
 
 template <int BITS, int CB, int NH>
@@ -2099,17 +2118,20 @@ __device__ __forceinline__ void pf_gemm(const void* codes, int32_t codes_s, int 
     const int nt = (nrows + 15) >> 4;                             // at most pf_nt<BITS>: the plan's pf_rows
     if constexpr (pf_nt<BITS>() == 7) {
         if (nt >= 7) {
-            pf_gemm_nt<BITS, CB, NH, 7>(EXL3C4_PF_ARGS);
+            pf_gemm_nt<BITS, CB, NH, 7, 1>(EXL3C4_PF_ARGS);
             return;
         }
     }
     switch (nt) {
-    case 1: pf_gemm_nt<BITS, CB, NH, 1>(EXL3C4_PF_ARGS); break;
-    case 2: pf_gemm_nt<BITS, CB, NH, 2>(EXL3C4_PF_ARGS); break;
-    case 3: pf_gemm_nt<BITS, CB, NH, 3>(EXL3C4_PF_ARGS); break;
-    case 4: pf_gemm_nt<BITS, CB, NH, 4>(EXL3C4_PF_ARGS); break;
-    case 5: pf_gemm_nt<BITS, CB, NH, 5>(EXL3C4_PF_ARGS); break;
-    default: pf_gemm_nt<BITS, CB, NH, 6>(EXL3C4_PF_ARGS); break;
+    case 1:
+        if (KC % 256 == 0) pf_gemm_nt<BITS, CB, NH, 1, 4>(EXL3C4_PF_ARGS);
+        else pf_gemm_nt<BITS, CB, NH, 1, 2>(EXL3C4_PF_ARGS);
+        break;
+    case 2: pf_gemm_nt<BITS, CB, NH, 2, 2>(EXL3C4_PF_ARGS); break;
+    case 3: pf_gemm_nt<BITS, CB, NH, 3, 2>(EXL3C4_PF_ARGS); break;
+    case 4: pf_gemm_nt<BITS, CB, NH, 4, 1>(EXL3C4_PF_ARGS); break;
+    case 5: pf_gemm_nt<BITS, CB, NH, 5, 1>(EXL3C4_PF_ARGS); break;
+    default: pf_gemm_nt<BITS, CB, NH, 6, 1>(EXL3C4_PF_ARGS); break;
     }
 #undef EXL3C4_PF_ARGS
 }
@@ -2122,7 +2144,7 @@ __device__ __forceinline__ void pf_gemm(const void* codes, int32_t codes_s, int 
 // narrower class's blocks past its width, are written zero; rows no run holds are the tail workgroups'.
 template <int BITS, int CB>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_gu_pf(const Exl3c4Launch a) {
-    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 2 * EXL3C4_PF_ROWS * PF_KP];
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * 2 * PF_BUF];
     constexpr int ACC_PITCH = 264;                                // floats: the epilogue's [48][256] with padding
     constexpr int EPI_T = 3;                                      // row tiles an epilogue pass (48 rows)
     static_assert(EPI_T * 16 * ACC_PITCH * 4 <= (int)sizeof(lds), "an epilogue pass fits the staging buffers");
@@ -2262,7 +2284,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 // in its block: a negative sorted_tok and a narrower class's tail as zero; with keep_sums the raw sums to dacc.
 template <int BITS, int CB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_dn_pf(const Exl3c4Launch a) {
-    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * EXL3C4_PF_ROWS * PF_KP];
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * PF_BUF];
     if (a.tail_from && (int)blockIdx.x >= a.tail_from) {          // the rows no run holds
         zero_dead_rows<4>(a, (int)blockIdx.x - a.tail_from);
         return;

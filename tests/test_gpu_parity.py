@@ -418,6 +418,17 @@ def test_launch_gather_gives_the_bits_of_the_launch_and_the_gather(torch_cuda, s
         assert np.array_equal(outs[0], oracle.moe_gather(want_y, True, w, row_of, nt, top_k))
 
 
+@pytest.mark.parametrize("geom,bits", [((256, 256), 4), ((384, 384), 3), ((640, 128), 8), ((128, 512), 2)])
+def test_prefill_chunks_of_every_tile_count(torch_cuda, geom, bits):
+    """Runs on both sides of each count of 16-row tiles a prefill chunk holds (its steps a stage follow the count), with
+    k an even and an odd number of 128-blocks in gate_up and in down: every op against the oracle."""
+    runs = (1, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 112, 113)
+    ids = np.repeat(np.arange(len(runs)), runs).astype(np.int32)[:, None]
+    case = Case(seed=700 + bits, n_tok=ids.shape[0], top_k=1, n_expert=len(runs), geoms=[geom], bits=bits, cb="mul1",
+                expert_ids=ids)
+    _check_all(case, f"tile counts {geom} K {bits}")
+
+
 @pytest.mark.parametrize("n_tok,top_k,n_expert,bits,dn_bits,cb", [
     (1, 4, 4, 4, 4, "mul1"), (1, 10, 40, 3, 6, "mul1"), (3, 10, 24, 5, 5, "mcg"), (7, 4, 6, 8, 8, "3inst"),
     (1, 31, 48, 2, 2, "mul1")])
