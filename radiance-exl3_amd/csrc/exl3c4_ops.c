@@ -38,13 +38,21 @@ static int64_t max_rows(const Exl3c4Op* o) {
     return m;
 }
 
-/* Rows a decode-path chunk holds at most: the least power of two >= min(M, 16). A token's top_k experts are distinct,
- * so an expert's run in a batch of M tokens holds at most M rows, and a chunk stages no more rows than a run can have
- * (at decode, M = 8: half the LDS of 16-row chunks). A routing that repeats an expert within a token makes longer runs;
- * they are cut into more chunks, with the same bits. */
-static int chunk_for(int64_t M) {
+/* Rows a decode-path chunk holds at most: the least power of two >= min(M, 4), or min(M, 16) where a token has one
+ * expert (a batch may then be one expert's, decoded once) or the launch is as large as the prefill path's. A token's
+ * top_k experts are distinct, so an expert's run in a batch of M tokens holds at most M rows, and a chunk stages no more
+ * rows than a run can have. Four: the launch's LDS follows the chunk's bound, not its rows, and the split-K count
+ * follows the LDS, while most runs here hold one or two rows -- 16-row chunks cost four splits of gate_up (2048 k) or
+ * eight (2560), each unit with its own start-up, sums and count, where 4-row chunks need one; a longer run is decoded
+ * once more for each further four rows, by more workgroups at once. Measured, chunks of 16 / 8 / 4 / 2 / 1 rows, the step
+ * in us (512 experts, top-10, K = 4): 32 tokens 130.7 / 123.5 / 121.3 / 125.4 / 139.1, with a Zipf popularity 106.9 /
+ * 99.2 / 96.6 / 111.5 / 136.0, hidden 2560 237.6 / 195.0 / 186.8 / 184.5 / 208.6; 16 tokens Zipf 73.6 / 68.8 / 64.9 /
+ * 69.0 / 76.1; top-2 of 8 experts, 16 tokens, 16 / 4 rows: 47.8 / 38.1; one expert's 16 rows 19.6 / 19.9. */
+#define CHUNK_ROWS_SPREAD 4
+static int chunk_for(const Exl3c4Op* o, int64_t T) {
+    const int cap = o->top_k >= 2 && T < exl3c4_prefill_min_rows(o->n_expert) ? CHUNK_ROWS_SPREAD : EXL3C4_CHUNK_ROWS;
     int c = 1;
-    while (c < EXL3C4_CHUNK_ROWS && c < M) c <<= 1;
+    while (c < cap && c < o->M) c <<= 1;
     return c;
 }
 
@@ -89,13 +97,13 @@ static int log2i(int v) {
 /* The prefill path (the rotation with the chunk plan, then one GEMM kernel a projection over chunks of up to 112 rows
  * of one expert) serves a launch of at least 64 sorted rows that average at least 7/8 of a row an expert: T >= 64 and
  * 8 T >= 7 n_expert (exl3c4_prefill_min_rows). Below it the decode kernels serve it (chunks of up to 16 rows, split-K;
- * gate_up_down as one kernel from EXL3C4_GD_FUSE_MIN_T rows). The rule is the crossover measured on MI355X at the
- * decode layer's experts (512 experts, 2048 / 512, K = 4, softmax top-10): gate_up_down by the decode kernels against
- * the prefill kernels, us a launch, M tokens (3 x 400 launches, alternating on one box): M = 26: 107.7 / 126.4,
- * 28: 113.9 / 128.2, 32: 127.6 / 131.0, 36: 139.6 / 152.0, 40: 151.5 / 156.5, 44: 155.5 / 157.8, 48: 169.1 / 160.8,
- * 56: 186.8 / 186.0 (an earlier build: 64: 204 / 191, 128: 302 / 264, 256: 389 / 285, 409: 491 / 293): the rule's
- * M >= 45 (T >= 448) sits between 44 and 48. The reference serves M >= 17 by its GEMM rows (kernels/exl3r4d/rows.c:
- * 255-315, kernels/exl3r4d/prefill.c:61-76); here the decode kernels keep the band below the crossover. A function of
+ * gate_up_down as one kernel from EXL3C4_GD_FUSE_MIN_T rows). The rule lies where neither routing loses much (measured on
+ * MI355X at the decode layer's experts, 512 experts, 2048 / 512, K = 4, top-10, the layer step in us by the decode
+ * kernels / by the prefill kernels): softmax routing M = 32: 122 / 135, 40: 144 / 159, 48: 157 / 162, 56: 173 / 184,
+ * 64: 187 / 185, 96: 238 / 211, 128: 269 / 235; a Zipf popularity 32: 97 / 103, 48: 135 / 110, 64: 173 / 132; hidden
+ * 2560 32: 188 / 188, 40: 215 / 219, 64: 305 / 276; 128 experts top-8 24: 72 / 79, 32: 79 / 81, 48: 96 / 83. The
+ * reference serves M >= 17 by its GEMM rows (kernels/exl3r4d/rows.c:255-315, kernels/exl3r4d/prefill.c:61-76); here the
+ * decode kernels keep the band below the crossover. A function of
  * T, n_expert and the op's widths (never of the routing): the prefill GEMMs address a chunk's staged rows by 32-bit
  * byte offsets (2 x 111 x pitch + 64 < 2^32), so an input pitch past EXL3C4_PF_MAX_PITCH halves (the caller's x, the
  * rotated input's 2 x cols, h's rows / 2) keeps the decode kernels at any T. */
@@ -161,7 +169,7 @@ static void carve(const Exl3c4Op* o, int64_t T, Carve* k) {
     memset(k, 0, sizeof *k);
     k->T = T;
     k->pf = prefill_path(o, T);
-    k->chunk = chunk_for(o->M);
+    k->chunk = chunk_for(o, T);
     int64_t off = 0;
     const int gu = op == EXL3C4_GATE_UP || op == EXL3C4_GU_DN;
     const int dn = op == EXL3C4_DOWN || op == EXL3C4_GU_DN;

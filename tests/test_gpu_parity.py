@@ -429,6 +429,18 @@ def test_prefill_chunks_of_every_tile_count(torch_cuda, geom, bits):
     _check_all(case, f"tile counts {geom} K {bits}")
 
 
+@pytest.mark.parametrize("runs,geom,bits", [
+    ((1, 3, 5), (384, 128), 3), ((4, 5, 8, 9), (256, 256), 4), ((2, 16, 6), (640, 384), 6)])
+def test_decode_chunks_at_the_edges_of_a_chunk(torch_cuda, runs, geom, bits):
+    """Runs on both sides of a decode chunk's rows (four where a token has two experts or more) and one run of every
+    token: the three-kernel and the one-kernel form by the row count, every op against the oracle."""
+    first = np.repeat(np.arange(len(runs)), runs).astype(np.int32)
+    ids = np.stack([first, np.full_like(first, len(runs))], 1)
+    case = Case(seed=800 + bits, n_tok=ids.shape[0], top_k=2, n_expert=len(runs) + 1, geoms=[geom], bits=bits, cb="mul1",
+                expert_ids=ids)
+    _check_all(case, f"decode runs {runs} K {bits}")
+
+
 @pytest.mark.parametrize("n_tok,top_k,n_expert,bits,dn_bits,cb", [
     (1, 4, 4, 4, 4, "mul1"), (1, 10, 40, 3, 6, "mul1"), (3, 10, 24, 5, 5, "mcg"), (7, 4, 6, 8, 8, "3inst"),
     (1, 31, 48, 2, 2, "mul1")])
