@@ -1144,24 +1144,31 @@ __device__ __forceinline__ void row_h(const Exl3c4Launch& a, int i, const GuRows
     if (threadIdx.x == 0) __hip_atomic_fetch_add(row_counter(a, i), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// gate_up_down in one launch (decode path). Workgroups g = 8 k + x (x < 8) take the sorted rows i = x (mod 8): first
-// every gate_up unit of those rows (row-major, the n_grp x ksplit units of k_gu), then every down unit (row-major, the
-// nblk blocks of k_dn). A gate_up unit of a chunk's row adds one to its counter once its sums are stored, and the last of
-// them forms the chunk's h (row_h) and adds one more; a down unit of that row waits for n_grp x ksplit + 1. The dispatcher deals workgroups to the 8 XCDs in turn and each XCD starts its
-// workgroups in order, so the workgroups g = x (mod 8) share one XCD (its L2 holds the row's sums) and when a down unit
-// runs, every gate_up unit before it has started; gate_up units never wait, so the waits end. The sums cross as
-// coherent accesses (part_ld / part_st), so the bits do not depend on where a workgroup lands. Built for 7 workgroups
-// a CU up to K = 6 (the register count it holds either way at K = 4; the schedule this target gives measured 0.5 us
-// faster); K = 7, 8 keep the looser target, under which they need no spill.
+// gate_up_down in one launch (decode path): first every gate_up unit (row-major, the n_grp x ksplit units of k_gu), then
+// every down unit (row-major, the nblk blocks of k_dn). A gate_up unit of a chunk's row adds one to its counter once its
+// sums are stored, and the last of them forms the chunk's h (row_h) and adds one more; a down unit of that row waits for
+// n_grp x ksplit + 1. The dispatcher deals workgroups to the 8 XCDs in turn and each XCD starts its workgroups in order,
+// so when a down unit runs, every gate_up unit of its XCD has started; gate_up units never wait, on any XCD, so the
+// waits end. The sums, h and the gathered y cross as coherent accesses (part_ld / part_st), so the bits do not depend on
+// where a workgroup lands.
+// From GD_SPREAD_T rows a row's units go to the XCDs in turn; below, row i's all to XCD i % 8 (workgroups g = 8 k + x
+// take the rows i = x (mod 8), gate_up units first). Which rows start a chunk follows the routing, so with a row an XCD
+// the XCDs' shares differ by a row or two of ten and the kernel ends with the fullest: the step in us by XCD / spread, 8
+// tokens 48.1 / 46.9, 16 tokens 77.6 / 75.6, 32 tokens 122.8 / 118.0, Zipf 8 and 32 tokens 45.6 / 43.8 and 96.5 / 91.7;
+// 1, 2 and 3 tokens 25.5 / 25.8, 28.2 / 29.1, 31.5 / 31.5 (a row's few units then meet in one L2).
+// Built for 7 workgroups a CU up to K = 6 (the register count it holds either way at K = 4; the schedule this target
+// gives measured 0.5 us faster); K = 7, 8 keep the looser target, under which they need no spill.
+constexpr int GD_SPREAD_T = 32;
 template <int BITS, int CB, int BD = BITS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BITS > BD ? BITS : BD) <= 6 ? 7 : 5, 8))) void k_gd(
     const Exl3c4Launch a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int xcd = (int)(blockIdx.x & 7), slot = (int)(blockIdx.x >> 3);
-    const int rows = xcd < a.T ? (a.T - 1 - xcd) / 8 + 1 : 0;
+    const int lg = a.T >= GD_SPREAD_T ? 0 : 3;                     // log2 of the lists the rows are dealt to
+    const int xcd = (int)blockIdx.x & ((1 << lg) - 1), slot = (int)(blockIdx.x >> lg);
+    const int rows = xcd < a.T ? ((a.T - 1 - xcd) >> lg) + 1 : 0;
     const int ugu = a.n_grp << a.ksplit_log2;
     if (slot < rows * ugu) {
-        const int i = xcd + 8 * (slot / ugu);
+        const int i = xcd + ((slot / ugu) << lg);
         const GuRows g = gu_unit<BITS, CB, true>(a, i, slot % ugu, a.lds_pitch_gu, lds);   // gate_up at K = BITS
         if (g.nrows > 0) {
             __shared__ int last_s;
@@ -1176,8 +1183,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BITS > BD 
         return;
     }
     const int d = slot - rows * ugu;
-    if (d < rows * a.nblk) dn_unit<BD, CB, true>(a, d % a.nblk, xcd + 8 * (d / a.nblk), lds);     // down at K = BD
-    else if (a.g_out) gather_empty(a, 8 * (d - rows * a.nblk) + xcd);  // the grid's last slots of each XCD
+    if (d < rows * a.nblk) dn_unit<BD, CB, true>(a, d % a.nblk, xcd + ((d / a.nblk) << lg), lds);     // down at K = BD
+    else if (a.g_out) gather_empty(a, ((d - rows * a.nblk) << lg) + xcd);  // each list's last slots
 }
 
 __global__ __launch_bounds__(256) void k_fill(int32_t* p, int64_t n) {
@@ -2557,9 +2564,10 @@ extern "C" int exl3c4_dev_gd(const Exl3c4Launch* a, void* stream, void* ev0, voi
     if (!f) return EXL3C4_E_DTYPE;
     if (a->T <= 0 || a->n_grp <= 0 || a->nblk <= 0) return 0;
     const uint32_t gu_lds = (uint32_t)(a->chunk_rows * a->lds_pitch_gu * 2), dn_lds = dn_lds_bytes(a);
-    const int64_t per_xcd = (int64_t)((a->T + 7) / 8) * (((int64_t)a->n_grp << a->ksplit_log2) + a->nblk) +
-                            (a->g_out ? (a->g_ntok + 31) / 32 : 0);  /* gather_empty: 4 tokens a workgroup */
-    return go2(f, dim3((unsigned)(8 * per_xcd)), (hipStream_t)stream, ev0, ev1, gu_lds > dn_lds ? gu_lds : dn_lds, *a);
+    const int lists = a->T >= GD_SPREAD_T ? 1 : 8;
+    const int64_t per_list = (int64_t)((a->T + lists - 1) / lists) * (((int64_t)a->n_grp << a->ksplit_log2) + a->nblk) +
+                             (a->g_out ? (a->g_ntok + 4 * lists - 1) / (4 * lists) : 0);  /* gather_empty: 4 tokens each */
+    return go2(f, dim3((unsigned)(lists * per_list)), (hipStream_t)stream, ev0, ev1, gu_lds > dn_lds ? gu_lds : dn_lds, *a);
 }
 
 // Instance state of the plugin rows (what a row's init hook allocates, never a launch): device memory zeroed once,
