@@ -1155,10 +1155,11 @@ __device__ __forceinline__ void row_h(const Exl3c4Launch& a, int i, const GuRows
 // take the rows i = x (mod 8), gate_up units first). Which rows start a chunk follows the routing, so with a row an XCD
 // the XCDs' shares differ by a row or two of ten and the kernel ends with the fullest: the step in us by XCD / spread, 8
 // tokens 48.1 / 46.9, 16 tokens 77.6 / 75.6, 32 tokens 122.8 / 118.0, Zipf 8 and 32 tokens 45.6 / 43.8 and 96.5 / 91.7;
-// 1, 2 and 3 tokens 25.5 / 25.8, 28.2 / 29.1, 31.5 / 31.5 (a row's few units then meet in one L2).
+// 56 rows of 384 and 256 widths at K = 8 50.5 / 45.0; 1, 2 and 3 tokens 25.5 / 25.8, 28.2 / 29.1, 31.5 / 31.5, 32 rows of
+// width 256 at K = 8 22.8 / 24.1, 40 rows 36.2 / 36.4 (a row's few units then meet in one L2).
 // Built for 7 workgroups a CU up to K = 6 (the register count it holds either way at K = 4; the schedule this target
 // gives measured 0.5 us faster); K = 7, 8 keep the looser target, under which they need no spill.
-constexpr int GD_SPREAD_T = 32;
+constexpr int GD_SPREAD_T = 40;
 template <int BITS, int CB, int BD = BITS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BITS > BD ? BITS : BD) <= 6 ? 7 : 5, 8))) void k_gd(
     const Exl3c4Launch a) {

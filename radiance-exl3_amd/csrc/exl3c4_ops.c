@@ -92,8 +92,14 @@ static int64_t chunk_bound(int64_t T, int64_t n_expert, int ch) {
  * units are many: the few of GU_UNITS_FEW and of one expert a token gain from the shorter unit all the same. The step
  * without / with the rule, us, 4 tokens: 2560 / 640 49.7 / 47.9, op by op 51.0 / 49.1; 1536 / 384 31.0 / 28.0. */
 static int even_split(int64_t nb, int s) { return 8 * ((nb + s - 1) / s * s - nb) <= nb; }
-static int ksplit_for(int64_t T, int64_t top_k, int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max, int ch) {
-    const int64_t units = T < GD_FUSE_ROWS && top_k >= 2 ? GU_UNITS_FEW : GU_UNITS;
+/* gate_up as a kernel of its own (gate_up alone, or a mixed pair of K that gate_up_down's single kernel does not carry)
+ * has no row chain behind a unit's start-up and takes more: 4096 / 5000 / 6500 units, the ops one by one, us: 12 tokens
+ * 70.7 / 67.1 / 67.0, 14 tokens of 384 and 256 widths 74.0 / 68.3 / 68.1, 14 tokens of top-6 over 128 experts of width 768
+ * 68.9 / 69.2 / 64.9 (5,088 units), but 8 tokens 51.9 / 51.9 / 53.6 and 16 tokens of width 256 34.8 / 34.6 / 36.9. */
+#define GU_UNITS_ALONE 5120
+static int ksplit_for(int64_t T, int64_t top_k, int alone, int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max,
+                      int ch) {
+    const int64_t units = top_k < 2 ? GU_UNITS : T < GD_FUSE_ROWS ? GU_UNITS_FEW : alone ? GU_UNITS_ALONE : GU_UNITS;
     const int many = T >= GD_FUSE_ROWS && top_k >= 2;
     int s = 1;
     while (s < 16 && 2 * s <= nb_min && chunks * n_grp * 2 * s <= units && (!many || even_split(nb_max, 2 * s))) s *= 2;
@@ -203,7 +209,8 @@ static void carve(const Exl3c4Op* o, int64_t T, Carve* k) {
         }
         int s = 1;
         if (!k->pf) {   /* split-K from T, M and the geometry: ksplit_for */
-            s = ksplit_for(T, o->top_k, chunk_bound(T, o->n_expert, k->chunk), rc / 128, nb_min, nb_max, k->chunk);
+            s = ksplit_for(T, o->top_k, op == EXL3C4_GATE_UP || !gd_pair(o), chunk_bound(T, o->n_expert, k->chunk),
+                           rc / 128, nb_min, nb_max, k->chunk);
             k->gu_lds_pitch = (int)(((nb_max + s - 1) / s) * 128 + 8);
         }
         k->split_gu = s;
