@@ -67,8 +67,8 @@ __global__ __launch_bounds__(256) void k_read_runs(const uint64_t* __restrict__ 
     if (lane == 0 && acc == 0x9E3779B9u) out[0] = acc;             // almost never: keeps the reads live
 }
 
-// The decode's VALU instructions in 8 independent chains a wave (the issue rate, not the latency): each round is the
-// mul1 pair sequence (2 v_pk_mul_lo_u16, 2 v_mad_u32_u16, v_sad_u8, v_sad_hi_u8, v_pk_fma_f16) on 8 register sets,
+// The VALU's issue rate on four-cycle instructions, in 8 independent chains a wave (not the latency): each round is the
+// mul1 pair by 16-bit products (2 v_pk_mul_lo_u16, 2 v_mad_u32_u16, v_sad_u8, v_sad_hi_u8, v_pk_fma_f16) on 8 sets,
 // 56 VALU instructions.
 __global__ __launch_bounds__(256) void k_valu(int rounds, uint32_t seed, uint32_t* out) {
     uint32_t r[8], y[8];

@@ -73,9 +73,14 @@ static int64_t chunk_bound(int64_t T, int64_t n_expert, int ch) {
  * gate_up unit) and adds a unit's fixed start-up; on configs[2] (80 chunks x 8 groups) S = 4, 2560 units against
  * about 1790 resident workgroups, measured 1.7 us a layer step faster than S = 2 (every unit resident at once) and
  * 5 us faster than S = 8. Then more splits while a split's staged rows would take more LDS than GU_LDS_BUDGET (which
- * keeps 7 workgroups a CU). */
+ * keeps 7 workgroups a CU). The limit, 4096 / 5000 / 6500 / 8200 units, the layer step in us: 8 tokens 47.2 / 47.2 / 51.6 /
+ * 51.6, 12 tokens 61.1 / 62.1 / 61.7 / 62.1, 16 tokens 76.4 / 75.5 / 76.7 / 77.3, 32 tokens 119.0 / 119.7 / 122.0 / 123.6,
+ * 16 tokens of width 256 33.3 / 33.5 / 38.7 / 38.4; the ops one by one 12 tokens 70.7 / 67.1 / 67.0 / 67.1, 14 tokens of
+ * widths 384 and 256 74.0 / 68.3 / 68.1 / 68.2, 14 tokens of top-6 over 128 experts of width 768 (5,088 units) 68.9 / 69.2 /
+ * 64.9 / 64.8, 8 tokens 51.9 / 51.9 / 53.6 / 53.5. One rule for gate_up and gate_up_down: the same splits, so that
+ * gate_up_down gives its pair's bits. */
 #ifndef GU_UNITS
-#define GU_UNITS 4096
+#define GU_UNITS 5120
 #endif
 #ifndef GU_LDS_BUDGET
 #define GU_LDS_BUDGET (20 * 1024)
@@ -92,14 +97,8 @@ static int64_t chunk_bound(int64_t T, int64_t n_expert, int ch) {
  * units are many: the few of GU_UNITS_FEW and of one expert a token gain from the shorter unit all the same. The step
  * without / with the rule, us, 4 tokens: 2560 / 640 49.7 / 47.9, op by op 51.0 / 49.1; 1536 / 384 31.0 / 28.0. */
 static int even_split(int64_t nb, int s) { return 8 * ((nb + s - 1) / s * s - nb) <= nb; }
-/* gate_up as a kernel of its own (gate_up alone, or a mixed pair of K that gate_up_down's single kernel does not carry)
- * has no row chain behind a unit's start-up and takes more: 4096 / 5000 / 6500 units, the ops one by one, us: 12 tokens
- * 70.7 / 67.1 / 67.0, 14 tokens of 384 and 256 widths 74.0 / 68.3 / 68.1, 14 tokens of top-6 over 128 experts of width 768
- * 68.9 / 69.2 / 64.9 (5,088 units), but 8 tokens 51.9 / 51.9 / 53.6 and 16 tokens of width 256 34.8 / 34.6 / 36.9. */
-#define GU_UNITS_ALONE 5120
-static int ksplit_for(int64_t T, int64_t top_k, int alone, int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max,
-                      int ch) {
-    const int64_t units = top_k < 2 ? GU_UNITS : T < GD_FUSE_ROWS ? GU_UNITS_FEW : alone ? GU_UNITS_ALONE : GU_UNITS;
+static int ksplit_for(int64_t T, int64_t top_k, int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max, int ch) {
+    const int64_t units = T < GD_FUSE_ROWS && top_k >= 2 ? GU_UNITS_FEW : GU_UNITS;
     const int many = T >= GD_FUSE_ROWS && top_k >= 2;
     int s = 1;
     while (s < 16 && 2 * s <= nb_min && chunks * n_grp * 2 * s <= units && (!many || even_split(nb_max, 2 * s))) s *= 2;
@@ -209,8 +208,7 @@ static void carve(const Exl3c4Op* o, int64_t T, Carve* k) {
         }
         int s = 1;
         if (!k->pf) {   /* split-K from T, M and the geometry: ksplit_for */
-            s = ksplit_for(T, o->top_k, op == EXL3C4_GATE_UP || !gd_pair(o), chunk_bound(T, o->n_expert, k->chunk),
-                           rc / 128, nb_min, nb_max, k->chunk);
+            s = ksplit_for(T, o->top_k, chunk_bound(T, o->n_expert, k->chunk), rc / 128, nb_min, nb_max, k->chunk);
             k->gu_lds_pitch = (int)(((nb_max + s - 1) / s) * 128 + 8);
         }
         k->split_gu = s;
