@@ -323,8 +323,8 @@ __device__ __forceinline__ half8_t as_half8(uint32_t a, uint32_t b, uint32_t c, 
 
 // gfx950's v_mfma_f32_16x16x32_f16 still reads its A and B registers for some cycles after it issues, and the compiler
 // does not hold back a VALU or load that writes them meanwhile (measured: an address computed into a just-issued MFMA's
-// B registers corrupted the product). Every step's MFMAs end with this guard: the scheduler may move nothing across
-// it, and its inputs keep the group's operand registers allocated through 16 wait states after the last MFMA.
+// B registers corrupted the product). Every tile's MFMAs end with this guard: the scheduler may move nothing across
+// it, and its inputs keep the tile's operand registers allocated through 16 wait states after the last MFMA.
 __device__ __forceinline__ void mfma_guard(const half8_t& a0, const half8_t& a1, const half8_t& b0, const half8_t& b1,
                                            const half8_t& b2, const half8_t& b3) {
     __builtin_amdgcn_sched_barrier(0);
@@ -2017,10 +2017,11 @@ __device__ __forceinline__ bool xcd_unit(int per, const int32_t* xb, const int32
 constexpr int PF_DYN_GU = 64, PF_DYN_DN = 0;
 
 // One k-step of the prefill GEMM: the step's B operands (decoded just before) against each of the chunk's NT row
-// tiles (4 MFMAs a tile), the step ending in mfma_guard: gfx950 does not interlock a VALU write against an in-flight
-// 16x16x32 MFMA's A/B reads, and the compiler does not pad for it. Between the tiles only LDS reads write A registers,
-// each issued behind the MFMAs that read the registers' last tile, and land well after those have read them. (A step's
-// decode and its MFMAs take
+// tiles (4 MFMAs a tile), each tile ending in mfma_guard, so that neither the LDS read of a later tile's A operands nor
+// a VALU value that the compiler puts into a tile's dead A registers (it moves part of the decode between the MFMAs)
+// comes within 16 wait states of the MFMAs that read them. One guard a step instead is 0.5% faster at 4096 tokens (578
+// against 583 us) and within the runs' spread elsewhere, and leaves such a write right behind its MFMA. (A step's decode
+// and its MFMAs take
 // their sum on a SIMD of 4 such waves, measured: the decode keeps the VALU pipe full and the MFMAs of the other waves
 // find no slot beside it; a step issued behind the next step's decode, or the waves split into a decoding and a
 // multiplying half each half-step, gained nothing.)
@@ -2035,9 +2036,10 @@ __device__ __forceinline__ void pf_step(const uint16_t* Ab, int kp, const uint32
     const half8_t b0 = as_half8(B[0], B[2], B[4], B[6]), b1 = as_half8(B[8], B[10], B[12], B[14]);
     const half8_t b2 = as_half8(B[1], B[3], B[5], B[7]), b3 = as_half8(B[9], B[11], B[13], B[15]);
     // The A operands of the next tile are read while this one multiplies, into a second set of registers where the tiles
-    // leave them (up to five; at six and seven the accumulators fill the 128 of 4 waves a SIMD). Measured against a read,
-    // a wait and a guard a tile, the layer step in us: 2048 tokens 410 -> 405, 4096 tokens 597 -> 586, 2560 / 640 at 1500
-    // tokens 526 -> 518, 4096 Zipf 661 -> 655. (32x32x16 MFMAs, half as many, measured slower: 620 against 574 at 4096.)
+    // leave them (up to five; at six and seven the accumulators fill the 128 of 4 waves a SIMD). Measured against a read
+    // and a wait a tile, the layer step in us: 2048 tokens 403.6 -> 397.8, 2560 / 640 at 1500 tokens 512.9 -> 507.9, 613
+    // tokens mcg K = 3 279.5 -> 277.3, 4096 tokens 583 -> 580. (32x32x16 MFMAs, half as many, measured slower: 620
+    // against 574 at 4096.)
     constexpr int AHEAD = NT <= 5 ? 1 : 0;
     half8_t Aa[AHEAD + 1], Ac[AHEAD + 1];
     Aa[0] = *(const half8_t*)Ab;
@@ -2055,14 +2057,12 @@ __device__ __forceinline__ void pf_step(const uint16_t* Ab, int kp, const uint32
         acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Aa[c], b1, acc[t][1], 0, 0, 0);
         acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ac[c], b2, acc[t][0], 0, 0, 0);
         acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Ac[c], b3, acc[t][1], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        mfma_guard(Aa[c], Ac[c], b0, b1, b2, b3);
         if (!AHEAD && t + 1 < NT) {
             Aa[0] = *(const half8_t*)next;
             Ac[0] = *(const half8_t*)(next + 8);
         }
     }
-    constexpr int last = (NT - 1) & AHEAD;
-    mfma_guard(Aa[last], Ac[last], b0, b1, b2, b3);
 }
 
 // The prefill GEMM of one chunk (<= EXL3C4_PF_ROWS rows of one expert) against the strips of one workgroup, all of k:

@@ -1,13 +1,16 @@
-"""The built gfx950 code object against the wait states an MFMA needs around VALU writes of its sources (no GPU).
+"""The built gfx950 code object against the wait states an MFMA needs around writes of its sources (no GPU).
 
-Two rules, in wait states (each instruction one, s_nop N counting N + 1), both of which the compiler's hazard
-recognizer enforces for the instructions it emits itself and for no inline-asm block's outputs:
+Three rules, in wait states (each instruction one, s_nop N counting N + 1). The compiler's hazard recognizer enforces the
+first two for the instructions it emits itself and for no inline-asm block's outputs, and the third not at all:
   RAW: a VALU write of a VGPR, then an MFMA that reads it as A, B or C: two wait states between them.
   WAR: an MFMA that reads a VGPR as C (accumulating into other registers), then a VALU write of that VGPR: three
        wait states between them (v_mfma_f32_16x16x32_f16 on gfx950; the compiler's own writes keep this spacing).
-A kernel whose asm writes break either can feed an MFMA a stale or a clobbered register, and whether it does depends
+  A/B: an MFMA that reads a VGPR as A or B, then a VALU write of that VGPR or the issue of an LDS or memory load into it:
+       16 wait states between them, what the kernels' guard behind each tile of MFMAs leaves (a write right behind the
+       MFMA has corrupted its product).
+A kernel whose writes break one can feed an MFMA a stale or a clobbered register, and whether it does depends
 on how the waves interleave. The decode keeps every asm write on a register the compiler itself defined just before
-(its own VALU write kept the spacing) and out of MFMA operands; this test holds both libraries to the two rules: it
+(its own VALU write kept the spacing) and out of MFMA operands; this test holds both libraries to the three rules: it
 unbundles each one's gfx950 code object, disassembles it, and walks from every MFMA within its straight-line code.
 """
 import os
@@ -22,6 +25,7 @@ LIBS = [os.path.join(ROOT, "radiance-exl3_amd", n) for n in ("libexl3c4.so", "li
 LLVM = "/opt/rocm/llvm/bin"
 NEED = 2          # wait states from a VALU write of a VGPR to an MFMA that reads it
 NEED_WAR = 3      # wait states from an MFMA that reads a VGPR as C (not its destination) to a VALU write of it
+NEED_AB = 16      # wait states from an MFMA that reads a VGPR as A or B to a VALU write of it or a load into it
 
 
 def _vregs(tok):
@@ -115,6 +119,32 @@ def war_violations(lines):
     return out
 
 
+def _load_dst(ins):
+    op, args = _operands(ins)
+    loads = op.startswith(("ds_read", "global_load", "flat_load", "scratch_load", "buffer_load"))
+    return _vregs(args[0]) if loads and "lds" not in ins.split() else set()
+
+
+def ab_violations(lines):
+    """A/B: (function, mfma line, writing line, wait states) for each VALU write of a VGPR, or load into one, that an MFMA
+    read as A or B fewer than NEED_AB wait states before."""
+    out, open_reads = [], []            # [mfma line, its A and B registers, wait states since]
+    for func, ins in _instructions(lines):
+        if ins is None:
+            open_reads = []
+            continue
+        op, args = _operands(ins)
+        d = _valu_dst(ins) | _load_dst(ins)
+        for m in open_reads:
+            if d & m[1]:
+                out.append((func, m[0], ins, m[2]))
+            m[2] += _wait_states(ins)
+        open_reads = [m for m in open_reads if m[2] < NEED_AB]
+        if op.startswith("v_mfma"):
+            open_reads.append([ins, _vregs(args[1]) | _vregs(args[2]), 0])
+    return out
+
+
 def _disassemble(tmp_path, lib):
     if not os.path.exists(lib):
         pytest.skip(f"{os.path.basename(lib)} is not built")
@@ -149,6 +179,30 @@ def test_the_rules_are_seen_on_planted_sequences():
     assert [v[3] for v in war_violations(war)] == [1]
     assert war_violations(war_ok) == [] and war_violations(in_place) == []
     assert war_violations([f, mf, "\ts_branch 0", "\tv_mov_b32_e32 v14, 0"]) == []
+
+
+def test_the_operand_read_rule_is_seen_on_planted_sequences():
+    """The A/B walk: a VALU write, an LDS read and a memory load into an MFMA's A or B registers right behind it or behind
+    its tile's other MFMAs (too soon), the same behind the guard (enough), and writes of other registers."""
+    f = "0000 <k>:"
+    mf = "\tv_mfma_f32_16x16x32_f16 v[10:13], v[44:47], v[48:51], v[10:13]"
+    other = "\tv_mfma_f32_16x16x32_f16 v[14:17], v[52:55], v[56:59], v[14:17]"
+    guard = ["\ts_nop 7", "\ts_nop 7"]
+    for w in ("\tv_mul_lo_u32 v44, v1, s17", "\tds_read_b128 v[44:47], v110 offset:2304",
+              "\tglobal_load_dwordx4 v[48:51], v[2:3], off"):
+        assert [v[3] for v in ab_violations([f, mf, w])] == [0]
+        assert [v[3] for v in ab_violations([f, mf, other, other, "\ts_waitcnt lgkmcnt(0)", w])] == [3]
+        assert ab_violations([f, mf] + guard + [w]) == []
+        assert ab_violations([f, mf, "\ts_endpgm", w]) == []
+    assert ab_violations([f, mf, "\tv_mul_lo_u32 v10, v1, s17", "\tds_read_b128 v[60:63], v44"]) == []
+
+
+@pytest.mark.parametrize("lib", LIBS, ids=[os.path.basename(p) for p in LIBS])
+def test_no_mfma_operand_is_overwritten_while_it_is_read(tmp_path, lib):
+    ab = ab_violations(_disassemble(tmp_path, lib))
+    for v in ab[:5]:
+        print(" | ".join(map(str, v)))
+    assert not ab, f"{len(ab)} writes of an MFMA's A or B registers fewer than {NEED_AB} wait states after it"
 
 
 @pytest.mark.parametrize("lib", LIBS, ids=[os.path.basename(p) for p in LIBS])
