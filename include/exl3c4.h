@@ -203,10 +203,18 @@ int exl3c4_launch_checked(const Exl3c4Op* op, void* scratch, int64_t scratch_byt
 int exl3c4_scratch_partials(const Exl3c4Op* op, int32_t gemm, int64_t* offset, int64_t* pitch, int64_t* split_stride,
                             int32_t* splits);
 
+/* exl3c4_launch_gather, whose single kernel's waiting down units leave their blocks to the unit that forms the row's h
+ * after `polls` polls (0 .. 128; a launch's own number is 128, more than one that runs alone needs): the same bits,
+ * by the path that a launch takes beside others. EXL3C4_E_INVAL for another `polls`. A checker's entry; no counterpart in
+ * the reference. */
+int exl3c4_launch_leaving(const Exl3c4Op* op, void* scratch, int64_t scratch_bytes, void* stream, void* ctr,
+                          int64_t ctr_bytes, const float* expert_w, const int32_t* row_of, void* out,
+                          int64_t out_pitch, int32_t polls);
+
 /* Where a launch of `op` that runs gate_up_down's single kernel leaves its status word in its scratch (an int32 at
- * scratch + *offset): 0 after a good launch; 1 when a down unit's wait for its row's gate_up units gave up (after
- * 0.5 s), and the output is then void. EXL3C4_E_INVAL when the launch does not run that kernel. A checker's entry;
- * no counterpart in the reference. */
+ * scratch + *offset): 0 after a good launch; 1 when the output is void -- the word was set before the launch, a row's
+ * counter was not zero before it, or a down unit's wait for its row's h gave up (after 0.5 s). EXL3C4_E_INVAL when the
+ * launch does not run that kernel. A checker's entry; no counterpart in the reference. */
 int exl3c4_scratch_status(const Exl3c4Op* op, int64_t* offset);
 
 /* W_hat of one stored weight [rows, cols] as fp16 bits [rows][w_pitch] on the device -- the same decode the GEMMs run,

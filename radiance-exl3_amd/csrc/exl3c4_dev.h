@@ -19,9 +19,16 @@ extern "C" {
 #define EXL3C4_STRIP 32
 #define EXL3C4_KSTEP 64
 /* int32 words between two row counters of gate_up_down's single kernel (256 B: each counter its own cache line), and
- * where in a row's line the count of its down units past their wait sits */
+ * where in a row's line the count of its down units past their wait sits. A row's counter is a u64: its gate_up units'
+ * count in the low EXL3C4_SYNC_COUNT bits, above them a bit for each of the row's 128-column blocks (up to
+ * EXL3C4_SYNC_BLOCKS) whose down unit left it to the unit that forms h. */
 #define EXL3C4_SYNC_STRIDE 64
 #define EXL3C4_SYNC_DONE 32
+#define EXL3C4_SYNC_COUNT 16
+#define EXL3C4_SYNC_BLOCKS (64 - EXL3C4_SYNC_COUNT)
+/* polls (0.3 us or more each) after which a waiting down unit leaves its block where it may: a launch that runs alone
+ * needed at most 44 (1 to 44 tokens, K 2..8, Zipf and even routing: waits of up to 20 us) */
+#define EXL3C4_LEAVE_POLLS 128
 /* Rows of one chunk on the prefill path at most: seven MFMA row tiles share each decoded step where a launch's K are
  * at most 4, six (EXL3C4_PF_ROWS_WIDE) at larger K. */
 #define EXL3C4_PF_ROWS 112
@@ -74,7 +81,7 @@ typedef struct Exl3c4Launch {
     const int32_t* sorted;
     const int32_t* off;
     int32_t*       plan;          /* prefill: [0] chunk count, then int4 {expert, row0, rows, 0} per chunk */
-    int32_t*       sync;          /* gate_up_down in one launch: a status word, then row i's counter at (i + 1) * SYNC_STRIDE */
+    int32_t*       sync;          /* gate_up_down in one launch: a status word, then row i's line at (i + 1) * SYNC_STRIDE */
     uint16_t*      hbuf;          /* gate_up_down in one launch: h (rotated, f16) of every chunk's rows [T][hbuf_pitch] */
     /* gate_up_down in one launch with moe_gather behind it (g_out non-null): out[t] = f16(sum over the token's slots
      * of expert_w x y[row_of]); token t's counter of 128-block b at g_ctr[t * SYNC_STRIDE + b] (zero, left zero) */
@@ -99,7 +106,10 @@ typedef struct Exl3c4Launch {
     int32_t        lds_pitch_gu;  /* gate_up_down in one launch: gate_up's staged row pitch (lds_pitch is down's) */
     int32_t        y_cols;
     int32_t        max_chunks;
-    int32_t        blk_per_wave;  /* gate_up's epilogue: 128-blocks of a row one wave takes */
+    union {
+        int32_t    blk_per_wave;  /* gate_up's epilogue: 128-blocks of a row one wave takes */
+        int32_t    leave_polls;   /* gate_up_down in one launch: polls after which a waiting down unit leaves */
+    };
     int32_t        keep_sums;     /* prefill: also leave the GEMMs' f32 sums in part / dacc (a checker's view) */
     int32_t        tail_from;     /* prefill GEMMs: nonzero asks for workgroups that zero the rows no run holds after
                                      the GEMM's (the launcher sets where they start) */

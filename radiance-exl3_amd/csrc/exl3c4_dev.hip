@@ -357,10 +357,10 @@ __device__ __forceinline__ int perm_slot(int k) {
 // with scalar loads. Holds a barrier: every thread of the workgroup calls it.
 struct Owner { int e, lo, hi; };
 constexpr int OWNER_LDS = 1024;
-__device__ Owner owner_wg(const Exl3c4Launch& a, int i) {
+__device__ __forceinline__ Owner owner_wg(const Exl3c4Launch& a, int i, int tid) {
     __shared__ int cnt_s[4];
     __shared__ int off_s[OWNER_LDS + 1];
-    const int n = a.n_expert, tid = (int)threadIdx.x;
+    const int n = a.n_expert;
     int cnt = 0;
     for (int e0 = 0; e0 <= n; e0 += 4 * 256) {                    // uniform trip count: ballots see every lane
         int o[4];
@@ -695,7 +695,7 @@ __device__ __forceinline__ GuRows gu_unit(const Exl3c4Launch& a, int i, int u, i
     const int grp = u >> a.ksplit_log2, split = u & (S - 1);
     // the chunk's sorted_tok (lane q: row i + q), read beside the owner search (taken by readlane below)
     const int tok_l = a.sorted[min(i + (lane & 15), a.T - 1)];
-    const Owner w = owner_wg(a, i);
+    const Owner w = owner_wg(a, i, (int)threadIdx.x);
     const int nrows = chunk_rows(a, w, i);
     if (!FUSED && u == 0 && threadIdx.x == 0) {
         a.row_info[2 * i] = w.e;
@@ -773,43 +773,78 @@ __global__ __launch_bounds__(256) void k_gepi(const Exl3c4Launch a) {
     }
 }
 
-// Row i's counter: each in its own cache line, so that polls and counts of different rows do not meet. Half a line on,
-// EXL3C4_SYNC_DONE words in, the count of the row's down units past their wait.
-__device__ __forceinline__ int32_t* row_counter(const Exl3c4Launch& a, int i) {
-    return a.sync + (int64_t)(i + 1) * EXL3C4_SYNC_STRIDE;
+// Row i's counter (exl3c4_dev.h): each in its own cache line, so that polls and counts of different rows do not meet.
+// Half a line on, EXL3C4_SYNC_DONE words in, the count of the row's down units past their wait.
+__device__ __forceinline__ uint64_t* row_counter(const Exl3c4Launch& a, int i) {
+    return (uint64_t*)(a.sync + (int64_t)(i + 1) * EXL3C4_SYNC_STRIDE);
+}
+__device__ __forceinline__ int32_t* row_done(const Exl3c4Launch& a, int i) {
+    return a.sync + (int64_t)(i + 1) * EXL3C4_SYNC_STRIDE + EXL3C4_SYNC_DONE;
+}
+__device__ __forceinline__ int count_of(uint64_t c) { return (int)(c & ((1u << EXL3C4_SYNC_COUNT) - 1u)); }
+
+// The output is void: bit 0 of the status word sync[0], and *fail, a flag the host can read without a synchronisation,
+// when the launch has one (the plugin rows' instances).
+__device__ __forceinline__ void set_status(const Exl3c4Launch& a) {
+    __hip_atomic_fetch_or(a.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (a.fail) __hip_atomic_store(a.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// How gate_up_down's single launch deals its rows' units to the XCDs: to all in turn (one list), or row i's all to XCD
+// i % 8 (eight lists; k_gd). One list only where a row's counter has a bit for each block, which its down units need to
+// leave (wait_gate_up).
+constexpr int GD_SPREAD_T = 40;
+__host__ __device__ __forceinline__ int gd_lists_log2(int64_t T, int nblk) {
+    return T >= GD_SPREAD_T && nblk <= EXL3C4_SYNC_BLOCKS ? 0 : 3;
 }
 
 // A down unit of gate_up_down's single launch waits here until its chunk's h is stored: row i's counter reaches
 // n_grp x ksplit + 1 (one count per gate_up unit of row i once its sums are stored, one more once the last of them has
-// formed h). The wait gives up after EXL3C4_WAIT_TICKS of the 100 MHz clock, or soon after another workgroup gave up,
-// and sets bit 0 of the status word sync[0] -- and *fail, a flag the host can read without a synchronisation, when
-// the launch has one (the plugin rows' instances) -- the output is then void; the launch still ends.
-// A status word already set when the wait begins also gives up at once, before any counter is read: a block whose
-// earlier launch gave up may hold stale counts (a late gate_up count lands after the row's down units zeroed the
-// row's counters), so every later launch on it is void and reports it again -- in the same launch -- until the
-// caller zeroes the block.
+// formed h). Every wait ends by itself, also beside another launch whose waiting units hold slots:
+// eight lists  the row's gate_up units precede this unit on its XCD, which starts a launch's workgroups in order: they
+//              have started, and a gate_up unit waits for nothing. (Beyond EXL3C4_WAIT_TICKS of the 100 MHz clock the
+//              wait gives up all the same and sets the status word.)
+// one list     a gate_up unit of the row may still need a slot on another XCD, and the units of another launch that wait
+//              there may need the slot this unit holds (a cycle of two launches). So a unit that has polled
+//              a.leave_polls times leaves block b to the unit that forms h: it sets b's bit in the row's counter and
+//              ends, and the count of h, an addition to the same word, hands that unit every bit set before it. A unit
+//              whose bit came after the count finds h ready in the value it read and goes on. So each block is run once,
+//              and no unit holds its slot for another's start.
+// A status word already set when the wait begins gives up at once, before any counter is read: a block whose earlier
+// launch gave up may hold stale counts (a late gate_up count lands after the row's down units zeroed the row's
+// counters), so every later launch on it is void and reports it again -- in the same launch -- until the caller zeroes
+// the block. A launch on a block that was not zero finds a count past the row's units (k_gd) and sets the status word.
+// False: the unit leaves (uniform in the workgroup).
 #define EXL3C4_WAIT_TICKS 50000000ull
-__device__ __forceinline__ void wait_gate_up(const Exl3c4Launch& a, int i) {
-    if (threadIdx.x == 0) {
+__device__ __forceinline__ bool wait_gate_up(const Exl3c4Launch& a, int i, int b, int tid) {
+    __shared__ int left_s;
+    const bool leaves = gd_lists_log2(a.T, a.nblk) == 0;          // uniform
+    if (tid == 0) {
         const int want = (a.n_grp << a.ksplit_log2) + 1;
-        const int32_t* cnt = row_counter(a, i);
+        uint64_t* cnt = row_counter(a, i);
         const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
         // the status word and the first poll go out together: no round trip more on the wait's path
         const int32_t st = __hip_atomic_load(a.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        int32_t c = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint64_t c = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         bool give_up = (st & 1) != 0;
-        for (unsigned n = 1; !give_up && c < want; ++n) {
+        int left = 0;
+        for (int n = 1; !give_up && count_of(c) < want; ++n) {
+            if (leaves && n > a.leave_polls) {
+                c = __hip_atomic_fetch_or(cnt, 1ull << (EXL3C4_SYNC_COUNT + b), __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+                left = count_of(c) < want;
+                break;
+            }
             __builtin_amdgcn_s_sleep(8);
             give_up = (n & 15) == 0 && ((__hip_atomic_load(a.sync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 1) ||
                                         __builtin_amdgcn_s_memrealtime() - t0 > EXL3C4_WAIT_TICKS);
             c = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (give_up) {
-            __hip_atomic_fetch_or(a.sync, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (a.fail) __hip_atomic_store(a.fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
+        if (give_up) set_status(a);
+        left_s = left;
     }
     __syncthreads();
+    return !leaves || !__builtin_amdgcn_readfirstlane(left_s);
 }
 
 // down, one workgroup per (sorted row i, 128-column output block b); the workgroup keyed on a chunk's first row takes
@@ -818,8 +853,8 @@ __device__ __forceinline__ void wait_gate_up(const Exl3c4Launch& a, int i) {
 // first: gate_up's h_rot = 1 output computed from gate_up's partial sums (gate_up_down), or the rows of x, rotated
 // (h_rot = 0) or as given (down alone). The raw accumulations also go to `dacc` (a checker's view of the sums before
 // any narrowing). Every (row, block) of y is written once: a row no run holds, a negative sorted_tok and a narrower
-// class's tail as zero. Inside gate_up_down's single launch (FUSED) the workgroup finds the row's owner itself and
-// waits for the row's gate_up units before it reads their sums.
+// class's tail as zero. Inside gate_up_down's single launch (FUSED) the workgroup finds the row's owner itself and, with
+// `wait`, waits for the row's h before it reads it, or leaves the block (wait_gate_up). tid: the thread's index.
 // y's 128-block b of one row: coherent stores when the launch gathers (the gathering unit may sit on another XCD and
 // reads them with coherent loads once every unit of the token's rows has counted, after its stores completed)
 __device__ __forceinline__ void put_y(const Exl3c4Launch& a, uint16_t* out, int lane, uint16_t v0, uint16_t v1) {
@@ -839,10 +874,10 @@ __device__ __forceinline__ void put_y(const Exl3c4Launch& a, uint16_t* out, int 
 // a token at most once (its slots name distinct experts), at most 16 rows at decode. Wave w takes rows w, w + 4, ..:
 // the row's count and its token's first 16 slots (rows and weights, lane u slot u) go out together, so a completing
 // count finds the slots in registers and the gather's first loads are the rows' y.
-__device__ void gather_count(const Exl3c4Launch& a, int i, int nrows, int b, int tok_l) {
+__device__ __forceinline__ void gather_count(const Exl3c4Launch& a, int i, int nrows, int b, int tok_l, int tid) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // this thread's y stores are done
     __syncthreads();                                              // ... and the workgroup's: the counts may go out
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = tid >> 6, lane = tid & 63;
     const int K = a.top_k;
     for (int q = wave; q < nrows; q += 4) {                       // k_gd: 4 waves a workgroup
         const int p = __builtin_amdgcn_readlane(tok_l, q);        // tok_l: sorted_tok of row i + lane
@@ -946,8 +981,8 @@ __device__ __forceinline__ void dn_stage_h(const Exl3c4Launch& a, int i, int nro
 }
 
 template <int BITS, int CB, bool FUSED>
-__device__ __forceinline__ void dn_unit(const Exl3c4Launch& a, int b, int i, unsigned char* lds) {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+__device__ __forceinline__ void dn_unit(const Exl3c4Launch& a, int b, int i, bool wait, int tid, unsigned char* lds) {
+    const int wave = tid >> 6, lane = tid & 63;
     // the chunk's sorted_tok (lane q: row i + q), read beside the owner search: the epilogue and the gather take it
     const int tok_l = a.sorted[min(i + (lane & 15), a.T - 1)];
     int e, nrows;
@@ -955,7 +990,7 @@ __device__ __forceinline__ void dn_unit(const Exl3c4Launch& a, int b, int i, uns
         e = __builtin_amdgcn_readfirstlane(a.row_info[2 * i]);
         nrows = __builtin_amdgcn_readfirstlane(a.row_info[2 * i + 1]);
     } else {
-        const Owner w = owner_wg(a, i);
+        const Owner w = owner_wg(a, i, tid);
         e = w.e;
         nrows = chunk_rows(a, w, i);
     }
@@ -975,7 +1010,7 @@ __device__ __forceinline__ void dn_unit(const Exl3c4Launch& a, int b, int i, uns
     if (b * 128 >= N) {                                           // a narrower class's tail
         for (int q = wave; q < nrows; q += 4)
             put_y(a, (uint16_t*)a.y + (int64_t)(i + q) * a.y_pitch + b * 128, lane, 0, 0);
-        if (FUSED && a.g_out) gather_count(a, i, nrows, b, tok_l);
+        if (FUSED && a.g_out) gather_count(a, i, nrows, b, tok_l, tid);
         return;
     }
     const int kp = a.lds_pitch;               // halves a staged row: k plus 8, so the 16 rows fall in different banks
@@ -992,15 +1027,14 @@ __device__ __forceinline__ void dn_unit(const Exl3c4Launch& a, int b, int i, uns
     const int el = had_col(lane), et = had_col_t(lane);          // the block's sums' columns, its outputs'
     const uint16_t sv0 = ldg16(svh, b * 128 + et), sv1 = ldg16(svh, b * 128 + 64 + et);
     const void* suh = (!a.h_from_gu && !a.h_rot) ? tab_entry(D.suh, D.suh_s, jx) : nullptr;
-    if (FUSED) wait_gate_up(a, i);
+    if (FUSED && wait && !wait_gate_up(a, i, b, tid)) return;
     // every down unit of the row has passed its wait once the row's last one counts here: that one zeroes the row's
     // counters at its end, so a launch leaves them as it found them (the reference's counter blocks,
     // kernels/exl3r4d/launch.c:311-324). Counted right after the wait, so the count's round trip runs under the
     // staging and the loop rather than at the unit's end.
     int done_old = 0;
-    if (FUSED && threadIdx.x == 0)
-        done_old = __hip_atomic_fetch_add(row_counter(a, i) + EXL3C4_SYNC_DONE, 1, __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
+    if (FUSED && tid == 0)
+        done_old = __hip_atomic_fetch_add(row_done(a, i), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
     // stage the chunk's rows
     const int nhb = KC / 128;
@@ -1108,22 +1142,23 @@ __device__ __forceinline__ void dn_unit(const Exl3c4Launch& a, int b, int i, uns
         const uint32_t yb = f2bf2(y0 * h2f(sv0), y1 * h2f(sv1));
         put_y(a, out, et, (uint16_t)yb, (uint16_t)(yb >> 16));
     }
-    if (FUSED && a.g_out) gather_count(a, i, nrows, b, tok_l);
-    if (FUSED && threadIdx.x == 0 && done_old == N / 128 - 1) {
-        __hip_atomic_store(row_counter(a, i), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(row_counter(a, i) + EXL3C4_SYNC_DONE, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (FUSED && a.g_out) gather_count(a, i, nrows, b, tok_l, tid);
+    if (FUSED && tid == 0 && done_old == N / 128 - 1) {
+        __hip_atomic_store(row_counter(a, i), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(row_done(a, i), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
 template <int BITS, int CB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_dn(const Exl3c4Launch a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    dn_unit<BITS, CB, false>(a, blockIdx.x, blockIdx.y, lds);
+    dn_unit<BITS, CB, false>(a, blockIdx.x, blockIdx.y, false, (int)threadIdx.x, lds);
 }
 
 // h of a chunk's rows (gate_up's epilogue with h_rot: had128, x svh, f16(silu(gate) * up), f16(had(f16(h * dn_suh))))
 // from the rows' partial sums, once, by the row's last gate_up unit: into hbuf, then one more count on row i's counter.
-__device__ __forceinline__ void row_h(const Exl3c4Launch& a, int i, const GuRows& g) {
+// Thread 0 returns the counter before it (the blocks left to this unit).
+__device__ __forceinline__ uint64_t row_h(const Exl3c4Launch& a, int i, const GuRows& g) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, el = had_col(lane);
     const int c = class_of(a, g.e);
     const int64_t jx = entry_of(a, g.e);
@@ -1141,51 +1176,91 @@ __device__ __forceinline__ void row_h(const Exl3c4Launch& a, int i, const GuRows
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_fetch_add(row_counter(a, i), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return threadIdx.x == 0 ? __hip_atomic_fetch_add(row_counter(a, i), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
 }
 
 // gate_up_down in one launch (decode path): first every gate_up unit (row-major, the n_grp x ksplit units of k_gu), then
 // every down unit (row-major, the nblk blocks of k_dn). A gate_up unit of a chunk's row adds one to its counter once its
-// sums are stored, and the last of them forms the chunk's h (row_h) and adds one more; a down unit of that row waits for
-// n_grp x ksplit + 1. The dispatcher deals workgroups to the 8 XCDs in turn and each XCD starts its workgroups in order,
-// so when a down unit runs, every gate_up unit of its XCD has started; gate_up units never wait, on any XCD, so the
-// waits end. The sums, h and the gathered y cross as coherent accesses (part_ld / part_st), so the bits do not depend on
-// where a workgroup lands.
+// sums are stored, and the last of them forms the chunk's h (row_h), adds one more and runs the blocks whose down units
+// left; a down unit of that row waits for n_grp x ksplit + 1, or leaves (wait_gate_up). The dispatcher deals workgroups
+// to the 8 XCDs in turn and each XCD starts its workgroups in order. The sums, h and the gathered y cross as coherent
+// accesses (part_ld / part_st), so the bits do not depend on where a workgroup lands.
 // From GD_SPREAD_T rows a row's units go to the XCDs in turn; below, row i's all to XCD i % 8 (workgroups g = 8 k + x
 // take the rows i = x (mod 8), gate_up units first). Which rows start a chunk follows the routing, so with a row an XCD
 // the XCDs' shares differ by a row or two of ten and the kernel ends with the fullest: the step in us by XCD / spread, 8
-// tokens 48.1 / 46.9, 16 tokens 77.6 / 75.6, 32 tokens 122.8 / 118.0, Zipf 8 and 32 tokens 45.6 / 43.8 and 96.5 / 91.7;
-// 56 rows of 384 and 256 widths at K = 8 50.5 / 45.0; 1, 2 and 3 tokens 25.5 / 25.8, 28.2 / 29.1, 31.5 / 31.5, 32 rows of
-// width 256 at K = 8 22.8 / 24.1, 40 rows 36.2 / 36.4 (a row's few units then meet in one L2).
+// tokens 46.25 / 44.4, K = 3 / 6 45.7 / 43.8, 16 tokens 76.6 / 75.7, 32 tokens 126.4 / 119.9, Zipf 8 and 32 tokens 44.3 /
+// 41.8 and 103.3 / 95.0, 56 rows of 384 and 256 widths at K = 8 45.4 / 40.3; on an earlier build 1, 2 and 3 tokens 25.5 /
+// 25.8, 28.2 / 29.1, 31.5 / 31.5, 32 rows of width 256 at K = 8 22.8 / 24.1, 40 rows 36.2 / 36.4 (a row's few units then
+// meet in one L2). The leaving costs nothing that was measured: without it 8 tokens took 44.9 us, 1 token 24.0 (24.16).
 // Built for 7 workgroups a CU up to K = 6 (the register count it holds either way at K = 4; the schedule this target
 // gives measured 0.5 us faster); K = 7, 8 keep the looser target, under which they need no spill.
-constexpr int GD_SPREAD_T = 40;
+typedef const __attribute__((address_space(4))) Exl3c4Launch* kernargs;
+// The argument block's cache lines into the scalar cache, all at once: the values a unit needs late are loaded where they
+// are used, each otherwise a miss of its own in a chain that nothing hides (a step of one token 25.4 -> 24.35 us).
+__device__ __forceinline__ void touch_kernargs(kernargs k) {
+    static_assert(EXL3C4_KERNARG_BYTES > 0x240 && EXL3C4_KERNARG_BYTES <= 0x280, "ten lines of 64 bytes");
+    uint32_t w;
+    asm volatile("s_load_dword %0, %1, 0x0\n\ts_load_dword %0, %1, 0x40\n\ts_load_dword %0, %1, 0x80\n\t"
+                 "s_load_dword %0, %1, 0xc0\n\ts_load_dword %0, %1, 0x100\n\ts_load_dword %0, %1, 0x140\n\t"
+                 "s_load_dword %0, %1, 0x180\n\ts_load_dword %0, %1, 0x1c0\n\ts_load_dword %0, %1, 0x200\n\t"
+                 "s_load_dword %0, %1, 0x240\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(w) : "s"(k));
+    asm volatile("" ::"s"(w));
+}
+
 template <int BITS, int CB, int BD = BITS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((BITS > BD ? BITS : BD) <= 6 ? 7 : 5, 8))) void k_gd(
     const Exl3c4Launch a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int lg = a.T >= GD_SPREAD_T ? 0 : 3;                     // log2 of the lists the rows are dealt to
+    kernargs ka = (kernargs)__builtin_amdgcn_kernarg_segment_ptr();    // a, where it lies
+    touch_kernargs(ka);
+    const int lg = gd_lists_log2(a.T, a.nblk);                     // log2 of the lists the rows are dealt to
     const int xcd = (int)blockIdx.x & ((1 << lg) - 1), slot = (int)(blockIdx.x >> lg);
     const int rows = xcd < a.T ? ((a.T - 1 - xcd) >> lg) + 1 : 0;
     const int ugu = a.n_grp << a.ksplit_log2;
-    if (slot < rows * ugu) {
-        const int i = xcd + ((slot / ugu) << lg);
+    int i, b, tid = (int)threadIdx.x;                              // down: block b of row i
+    uint64_t more = 0;                                             // ... and the row's further blocks to run
+    const bool gu = slot < rows * ugu;
+    if (gu) {
+        i = xcd + ((slot / ugu) << lg);
         const GuRows g = gu_unit<BITS, CB, true>(a, i, slot % ugu, a.lds_pitch_gu, lds);   // gate_up at K = BITS
-        if (g.nrows > 0) {
-            __shared__ int last_s;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this thread's sums are stored
-            __syncthreads();
-            if (threadIdx.x == 0)
-                last_s = __hip_atomic_fetch_add(row_counter(a, i), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                         ugu - 1;
-            __syncthreads();
-            if (last_s) row_h(a, i, g);                                // the row's last gate_up unit forms h
+        if (g.nrows == 0) return;
+        __shared__ uint64_t word_s;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // this thread's sums are stored
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            word_s = __hip_atomic_fetch_add(row_counter(a, i), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (count_of(word_s) >= ugu) set_status(a);                // more counts than units: the block was not zero
         }
-        return;
+        __syncthreads();
+        if (count_of(word_s) != ugu - 1) return;
+        const uint64_t w = row_h(a, i, g);                             // the row's last gate_up unit forms h
+        if (threadIdx.x == 0) word_s = w >> EXL3C4_SYNC_COUNT;
+        __syncthreads();
+        more = word_s;                                                 // and runs the blocks whose down units left
+        if (a.nblk < EXL3C4_SYNC_BLOCKS) more &= (1ull << a.nblk) - 1ull;   // never a block past y's, whatever the word held
+        if (more == 0) return;
+        b = __builtin_ctzll(more);
+        more &= more - 1;
+        __syncthreads();
+    } else {
+        const int d = slot - rows * ugu;
+        if (d >= rows * a.nblk) {
+            if (a.g_out) gather_empty(a, ((d - rows * a.nblk) << lg) + xcd);  // each list's last slots
+            return;
+        }
+        i = xcd + ((d / a.nblk) << lg);
+        b = d % a.nblk;
     }
-    const int d = slot - rows * ugu;
-    if (d < rows * a.nblk) dn_unit<BD, CB, true>(a, d % a.nblk, xcd + ((d / a.nblk) << lg), lds);     // down at K = BD
-    else if (a.g_out) gather_empty(a, ((d - rows * a.nblk) << lg) + xcd);  // each list's last slots
+    for (;;) {
+        dn_unit<BD, CB, true>(*(const Exl3c4Launch*)ka, b, i, !gu, tid, lds);   // down at K = BD
+        if (more == 0) return;
+        b = __builtin_ctzll(more);
+        more &= more - 1;
+        // the next block's values are formed anew: kept across the loop they would take its registers (28 spilled)
+        asm volatile("" : "+v"(tid), "+s"(ka), "+s"(i));
+        __syncthreads();
+    }
 }
 
 __global__ __launch_bounds__(256) void k_fill(int32_t* p, int64_t n) {
@@ -2586,7 +2661,7 @@ extern "C" int exl3c4_dev_gd(const Exl3c4Launch* a, void* stream, void* ev0, voi
     if (!f) return EXL3C4_E_DTYPE;
     if (a->T <= 0 || a->n_grp <= 0 || a->nblk <= 0) return 0;
     const uint32_t gu_lds = (uint32_t)(a->chunk_rows * a->lds_pitch_gu * 2), dn_lds = dn_lds_bytes(a);
-    const int lists = a->T >= GD_SPREAD_T ? 1 : 8;
+    const int lists = 1 << gd_lists_log2(a->T, a->nblk);
     const int64_t per_list = (int64_t)((a->T + lists - 1) / lists) * (((int64_t)a->n_grp << a->ksplit_log2) + a->nblk) +
                              (a->g_out ? (a->g_ntok + 4 * lists - 1) / (4 * lists) : 0);  /* gather_empty: 4 tokens each */
     return go2(f, dim3((unsigned)(lists * per_list)), (hipStream_t)stream, ev0, ev1, gu_lds > dn_lds ? gu_lds : dn_lds, *a);

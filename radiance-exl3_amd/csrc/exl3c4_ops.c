@@ -440,7 +440,8 @@ static void base_args(const Exl3c4Op* o, const Carve* k, char* s, Exl3c4Launch* 
 /* How a launch runs: the events of a timed launch go to exactly one kernel of the sequence; keep_sums has the
  * prefill GEMMs also write their f32 sums to scratch (exl3c4_launch_checked); ctr: gate_up_down's counter block from
  * the caller (exl3c4_launch_ctr), or null; gx: moe_gather riding in gate_up_down's single kernel
- * (exl3c4_launch_gather), or null; fail: a host-visible flag the single kernel sets when a wait gives up, or null. */
+ * (exl3c4_launch_gather), or null; fail: a host-visible flag the single kernel sets when its output is void, or null;
+ * leave: one more than the polls after which the single kernel's waiting down units leave, or 0 for its own number. */
 typedef struct {
     const float*   w;
     const int32_t* row_of;
@@ -454,6 +455,7 @@ typedef struct Ctx {
     int32_t*      ctr;
     const Gather* gx;
     int32_t*      fail;
+    int           leave;
 } Ctx;
 #define EV(k) (t->kernel == (k) ? t->ev0 : NULL), (t->kernel == (k) ? t->ev1 : NULL)
 
@@ -532,6 +534,7 @@ static int launch_gd1(const Exl3c4Op* o, const Carve* k, char* s, void* stream, 
     g.hbuf = (uint16_t*)(s + k->h);
     g.hbuf_pitch = (int32_t)k->h_pitch;
     g.fail = t->fail;
+    g.leave_polls = t->leave ? t->leave - 1 : EXL3C4_LEAVE_POLLS;
     if (t->ctr) {                                 /* the caller's counter block: zero, and left zero */
         g.sync = t->ctr;
     } else {
@@ -651,12 +654,12 @@ static int launch_impl(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, 
 }
 
 int exl3c4_launch(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream) {
-    const Ctx t = { -1, NULL, NULL, 0, NULL, NULL, NULL };
+    const Ctx t = { -1, NULL, NULL, 0, NULL, NULL, NULL, 0 };
     return launch_impl(o, scratch, scratch_bytes, stream, &t);
 }
 
 int exl3c4_launch_checked(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream) {
-    const Ctx t = { -1, NULL, NULL, 1, NULL, NULL, NULL };
+    const Ctx t = { -1, NULL, NULL, 1, NULL, NULL, NULL, 0 };
     return launch_impl(o, scratch, scratch_bytes, stream, &t);
 }
 
@@ -682,7 +685,7 @@ int exl3c4_launch_inst(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, 
     if (k.gd1 && ctr && (ctr_bytes < (o->T + 1) * EXL3C4_SYNC_STRIDE * 4 || (uintptr_t)ctr % 256))
         return EXL3C4_E_SCRATCH;
     const int one = k.gd1 || gd_few(o, &k, ctr, ctr_bytes, (o->T + 1) * EXL3C4_SYNC_STRIDE * 4);
-    const Ctx t = { -1, NULL, NULL, 0, one ? (int32_t*)ctr : NULL, NULL, fail };
+    const Ctx t = { -1, NULL, NULL, 0, one ? (int32_t*)ctr : NULL, NULL, fail, 0 };
     return launch_impl(o, scratch, scratch_bytes, stream, &t);
 }
 
@@ -691,8 +694,9 @@ int exl3c4_launch_ctr(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, v
     return exl3c4_launch_inst(o, scratch, scratch_bytes, stream, ctr, ctr_bytes, NULL);
 }
 
-int exl3c4_launch_gather(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream, void* ctr,
-                         int64_t ctr_bytes, const float* expert_w, const int32_t* row_of, void* out, int64_t out_pitch) {
+static int launch_gather(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream, void* ctr,
+                         int64_t ctr_bytes, const float* expert_w, const int32_t* row_of, void* out, int64_t out_pitch,
+                         int leave) {
     int rc;
     if (!o) return EXL3C4_E_INVAL;
     if ((rc = check(o)) != EXL3C4_OK) return rc;
@@ -710,13 +714,25 @@ int exl3c4_launch_gather(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes
     if (fuse && (ctr_bytes < all_ctr || (uintptr_t)ctr % 256)) return EXL3C4_E_SCRATCH;
     if (k.gd1 && ctr && !fuse && (ctr_bytes < rows_ctr || (uintptr_t)ctr % 256)) return EXL3C4_E_SCRATCH;
     const Gather gx = { expert_w, row_of, out, out_pitch };
-    const Ctx tf = { -1, NULL, NULL, 0, (int32_t*)ctr, &gx, NULL };
+    const Ctx tf = { -1, NULL, NULL, 0, (int32_t*)ctr, &gx, NULL, leave };
     if (fuse) return launch_impl(o, scratch, scratch_bytes, stream, &tf);
     const int one = k.gd1 || gd_few(o, &k, ctr, ctr_bytes, rows_ctr);
-    const Ctx t = { -1, NULL, NULL, 0, one ? (int32_t*)ctr : NULL, NULL, NULL };
+    const Ctx t = { -1, NULL, NULL, 0, one ? (int32_t*)ctr : NULL, NULL, NULL, leave };
     if ((rc = launch_impl(o, scratch, scratch_bytes, stream, &t)) != EXL3C4_OK) return rc;
     return exl3c4_moe_gather(o->y, EXL3C4_BF16, o->y_pitch, expert_w, row_of, o->M, o->top_k, o->y_cols, out,
                              out_pitch, stream);
+}
+
+int exl3c4_launch_gather(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream, void* ctr,
+                         int64_t ctr_bytes, const float* expert_w, const int32_t* row_of, void* out, int64_t out_pitch) {
+    return launch_gather(o, scratch, scratch_bytes, stream, ctr, ctr_bytes, expert_w, row_of, out, out_pitch, 0);
+}
+
+int exl3c4_launch_leaving(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream, void* ctr,
+                          int64_t ctr_bytes, const float* expert_w, const int32_t* row_of, void* out, int64_t out_pitch,
+                          int32_t polls) {
+    if (polls < 0 || polls > EXL3C4_LEAVE_POLLS) return EXL3C4_E_INVAL;
+    return launch_gather(o, scratch, scratch_bytes, stream, ctr, ctr_bytes, expert_w, row_of, out, out_pitch, polls + 1);
 }
 
 int exl3c4_launch_timed(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream, int32_t kernel,
@@ -727,7 +743,7 @@ int exl3c4_launch_timed(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes,
     Carve k;
     carve(o, o->T, &k);
     if (!runs_kernel(o, &k, kernel)) return EXL3C4_E_INVAL;
-    const Ctx t = { kernel, ev_start, ev_stop, 0, NULL, NULL, NULL };
+    const Ctx t = { kernel, ev_start, ev_stop, 0, NULL, NULL, NULL, 0 };
     return launch_impl(o, scratch, scratch_bytes, stream, &t);
 }
 

@@ -94,6 +94,8 @@ def lib():
         L.exl3c4_launch_ctr.argtypes = [C.POINTER(Op), _p, _i64, _p, _p, _i64]
         L.exl3c4_launch_gather.restype = C.c_int
         L.exl3c4_launch_gather.argtypes = [C.POINTER(Op), _p, _i64, _p, _p, _i64, _p, _p, _p, _i64]
+        L.exl3c4_launch_leaving.restype = C.c_int
+        L.exl3c4_launch_leaving.argtypes = [C.POINTER(Op), _p, _i64, _p, _p, _i64, _p, _p, _p, _i64, _i32]
         L.exl3c4_scratch_status.restype = C.c_int
         L.exl3c4_scratch_status.argtypes = [C.POINTER(Op), C.POINTER(_i64)]
         L.exl3c4_record_to_codes.restype = C.c_int
@@ -380,6 +382,14 @@ def launch_gather(o: Op, scratch, ctr, w, row_of, out, stream=None) -> int:
     m = 0 if ctr is None else ctr.numel()
     return int(lib().exl3c4_launch_gather(C.byref(o), _ptr(scratch), n, _stream(stream), _ptr(ctr), m, _ptr(w),
                                           _ptr(row_of), _ptr(out), out.stride(0)))
+
+
+def launch_leaving(o: Op, scratch, ctr, w, row_of, out, polls: int, stream=None) -> int:
+    """exl3c4_launch_leaving: launch_gather, the single kernel's waiting down units leaving after `polls` polls."""
+    n = 0 if scratch is None else scratch.numel()
+    m = 0 if ctr is None else ctr.numel()
+    return int(lib().exl3c4_launch_leaving(C.byref(o), _ptr(scratch), n, _stream(stream), _ptr(ctr), m, _ptr(w),
+                                           _ptr(row_of), _ptr(out), out.stride(0), polls))
 
 
 def partial_sums(o: Op, scratch, gemm: int = 0):
