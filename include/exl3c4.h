@@ -241,7 +241,8 @@ int exl3c4_router_topk(const void* logits, int32_t logits_dtype, int64_t n_tok, 
  * sort (include/exl3_abi.h:109-123): expert_offset i32 [n_expert + 1] (expert e's rows [off[e], off[e+1]), off[n_expert]
  * the live count), sorted_tok i32 [T] (-1 past the live count), and, when not null, expert_count i32 [n_expert] and
  * row_of i32 [T] (the sorted row of pair p, -1 for a dropped pair: what the gather reads). A pair whose expert is
- * outside [expert_base, expert_base + n_expert) is dropped. n_expert <= 1024. */
+ * outside [expert_base, expert_base + n_expert) is dropped. n_expert <= 1024. row_of may be expert_ids itself (then one
+ * workgroup does it all). */
 int exl3c4_moe_scatter(const int32_t* expert_ids, int64_t n_tok, int32_t top_k, int64_t expert_base,
                        int64_t n_expert, int32_t* sorted_tok, int32_t* expert_offset, int32_t* expert_count,
                        int32_t* row_of, void* stream);

@@ -470,8 +470,11 @@ extern "C" int exl3c4_dev_router(const void* logits, int32_t dtype, int64_t n_to
 
 extern "C" int exl3c4_dev_scatter(const int32_t* ids, int64_t T, int64_t base, int32_t n_expert, int32_t* sorted,
                                   int32_t* off, int32_t* count, int32_t* row_of, void* stream) {
-    // a workgroup each SC_SEG pairs, up to one a CU (a segment is then several SC_SEG); one when there is no pair
-    const int64_t segs = T > 0 ? (T + SC_SEG - 1) / SC_SEG : 1, per = (segs + SC_MAX_WG - 1) / SC_MAX_WG;
+    // a workgroup each SC_SEG pairs, up to one a CU (a segment is then several SC_SEG); one when there is no pair, and one
+    // when row_of is written over ids: it has counted every pair before it writes any, and reads a later segment's ids
+    // before that segment's rows go out, while other workgroups would still be counting
+    const int64_t segs = T > 0 ? (T + SC_SEG - 1) / SC_SEG : 1;
+    const int64_t per = row_of == ids ? segs : (segs + SC_MAX_WG - 1) / SC_MAX_WG;
     const unsigned wgs = (unsigned)((segs + per - 1) / per);
     hipLaunchKernelGGL(k_scatter, dim3(wgs), dim3(SC_THREADS), 0, (hipStream_t)stream, ids, (uint32_t)T, base,
                        n_expert, (uint32_t)(per * SC_SEG), sorted, off, count, row_of);

@@ -110,6 +110,25 @@ def test_scatter_segments_match_the_oracle(torch_cuda, n_tok, top_k, n_expert, l
         assert np.array_equal(g, w_), name
 
 
+@pytest.mark.parametrize("n_tok,top_k,n_expert", [(8, 10, 512), (300, 1, 7), (2048, 10, 512), (4096, 10, 512)])
+def test_scatter_writes_row_of_over_the_ids(torch_cuda, n_tok, top_k, n_expert):
+    """row_of the same buffer as expert_ids: each pair's row in the place of its expert, the other outputs as with a buffer
+    of its own, several times over (no pair is counted after a row was written)."""
+    import exl3c4
+    import oracle
+    torch = torch_cuda
+    ids = np.random.default_rng(n_tok).integers(0, n_expert, (n_tok, top_k)).astype(np.int32)
+    want = oracle.moe_scatter_full(ids, n_expert, 0)
+    for _ in range(5):
+        io = torch.from_numpy(ids.copy()).cuda()
+        st = torch.zeros(n_tok * top_k, dtype=torch.int32, device="cuda")
+        off, cnt = (torch.zeros(n_expert + k, dtype=torch.int32, device="cuda") for k in (1, 0))
+        assert exl3c4.moe_scatter(io, n_expert, st, off, cnt, io, 0) == 0
+        torch.cuda.synchronize()
+        for g, w_, name in zip((st, off, cnt, io), want, ("sorted_tok", "expert_offset", "expert_count", "row_of")):
+            assert np.array_equal(g.cpu().numpy().reshape(-1), w_), name
+
+
 @pytest.mark.parametrize("n_tok,E,top_k", [(8, 512, 10), (16, 512, 10), (40, 512, 10), (16, 8, 4), (16, 1024, 64),
                                             (3, 1, 1), (16, 64, 64), (5, 100, 7)])
 def test_router_topk_scatter_matches_the_oracle(torch_cuda, n_tok, E, top_k):
