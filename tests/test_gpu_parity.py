@@ -364,9 +364,9 @@ def test_gate_up_down_with_a_counter_block_leaves_it_zero_and_gives_the_same_bit
     (81, 6, 8, 40, [(512, 256), (256, 128)], 0.0, False),       # two classes: the narrower one's blocks are zero
     (82, 8, 10, 128, [(512, 256)], 0.0, True),                  # a token whose slots all drop
     (83, 5, 8, 12, [(256, 128)], 0.1, False),                   # few experts: chunks of several rows
-    (84, 2, 8, 12, [(256, 128)], 0.0, False),                   # T = 16: two kernels, then the gather's own
-    (85, 1, 2, 4, [(256, 128), (512, 256)], 0.0, False),       # T = 2: the smallest h formed by the epilogue kernel
-    (86, 3, 10, 16, [(512, 256)], 0.2, False),                  # T = 30, the largest below the one-kernel form
+    (84, 2, 8, 12, [(256, 128)], 0.0, False),                   # T = 16, eight experts a token: one kernel as well
+    (85, 1, 2, 4, [(256, 128), (512, 256)], 0.0, False),       # T = 2, two a token: three kernels, the gather's own
+    (86, 3, 10, 16, [(512, 256)], 0.2, False),                  # T = 30: one kernel as well
 ])
 def test_launch_gather_gives_the_bits_of_the_launch_and_the_gather(torch_cuda, seed, n_tok, top_k, n_expert, geoms,
                                                                    drop, empty):
@@ -464,6 +464,52 @@ def test_few_rows_with_a_counter_block_run_as_one_kernel(torch_cuda, n_tok, top_
         torch.cuda.synchronize()
         assert np.array_equal(y.cpu().numpy().view(np.uint16), want)
         assert bool((ctr.view == (0x5A if small else 0)).all()) and ctr.ok()
+
+
+@pytest.mark.parametrize("n_tok,top_k,lines,reads", [
+    (2, 8, 0, False),                                           # no block: three kernels, then the gather's own
+    (5, 3, 64, False),                                          # fewer than four experts a token: as without a block
+    (15, 2, 64, False),
+    (2, 8, 16, False),                                          # a line short of the status word and the rows' counters
+    (2, 8, 17, True),                                           # the rows' alone: one kernel, then the gather's own
+    (3, 10, 33, True),                                          # a line short of the gather's
+    (3, 10, 34, True),                                          # all of them: the gather in the kernel
+])
+def test_launch_gather_below_32_rows_by_its_counter_block(torch_cuda, n_tok, top_k, lines, reads):
+    """exl3c4_launch_gather of 15 to 30 rows, with a counter block of `lines` lines of 256 bytes: y and out bit for bit
+    those of exl3c4_launch and exl3c4_moe_gather; a block that the launch is not to read (its bytes anything) stays as it
+    was, one that it reads (zero) is left zero."""
+    import exl3c4 as ex
+    import oracle
+    torch = torch_cuda
+    n_expert = 12 if top_k <= 8 else 16
+    case = Case(seed=620 + 10 * n_tok + top_k, n_tok=n_tok, top_k=top_k, n_expert=n_expert, geoms=[(512, 256)], bits=4,
+                cb="mul1")
+    dev = Dev(case)
+    assert 2 <= case.T < ex.GD_FUSE_MIN_T
+    N = max(d["rows"] for d in dev.tabs["dn"])
+    _, _, _, row_of = oracle.moe_scatter_full(case.ids, n_expert)
+    w = torch.from_numpy(np.random.default_rng(621).random((n_tok, top_k)).astype(np.float32)).cuda()
+    rt = torch.from_numpy(row_of).cuda()
+    got = []
+    for gather in (False, True):
+        y, out = dev.out(N, fill=0x1234), dev.out(N, fill=0x1234, rows=n_tok)
+        o = dev.gd_op(y)
+        s = dev.scratch(o)
+        print(f"launch_gather T {case.T} lines {lines} gather {gather}", flush=True)
+        if gather:
+            fill = 0 if reads else 0x5A
+            ctr = dev.guard(256 * lines, fill=fill) if lines else None
+            assert ex.launch_gather(o, s, ctr.view if lines else None, w, rt, out) == 0
+            torch.cuda.synchronize()
+            assert not lines or (bool((ctr.view == fill).all()) and ctr.ok())
+        else:
+            assert ex.launch(o, s) == 0 and ex.moe_gather(y, True, w, rt, out) == 0
+            torch.cuda.synchronize()
+        got.append((y.cpu().numpy().view(np.uint16), out.cpu().numpy().view(np.uint16)))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    assert np.array_equal(got[0][0], dev.gate_up_down())
+    dev.check_guards(f"launch_gather T {case.T} lines {lines}")
 
 
 def test_launch_gather_with_rows_past_t_leaves_the_counter_block_good(torch_cuda):
