@@ -680,7 +680,7 @@ __device__ __forceinline__ void gu_stage(const Exl3c4Launch& a, int i, int nrows
 }
 
 // gate_up's GEMM: one workgroup per (sorted row i, group of four 32-column strips, k split). The workgroup keyed on
-// a chunk's first row takes the chunk (at most 16 rows); the others leave. Its four waves take the group's four
+// a chunk's first row takes the chunk (at most a.chunk_rows rows); the others leave. Its four waves take the group's four
 // strips over the split's 128-blocks of k; the split's input rows -- rotated here, f16(had128(f16(x * suh or suh1)))
 // of the token's row, or read as given (a_rot) -- are staged once in LDS for all four. The strip's sums go to
 // part[split][row][col]; their consumer adds the splits in a fixed order, so the bits do not depend on scheduling.
@@ -1086,26 +1086,14 @@ __device__ __forceinline__ void dn_unit(const Exl3c4Launch& a, int b, int i, boo
         const int64_t r = i + q;
         for (int hb = wave; hb < nhb; hb += 4) {
             uint16_t v0 = 0, v1 = 0;
-            int ep = el;                                          // where the staged values go
             if (FUSED) {                                          // the row's h, formed once (row_h)
                 const uint16_t* hs = a.hbuf + r * a.hbuf_pitch + hb * 128;
                 v0 = __hip_atomic_load(hs + el, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 v1 = __hip_atomic_load(hs + el + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else if (a.h_from_gu) {
-                if (a.sorted[r] >= 0) gate_up_block<false>(a, a.cls[c], r, hb, jx, 1, lane, v0, v1);
-            } else {
-                const void* xs = (const uint16_t*)a.x + r * a.x_pitch + hb * 128;
-                const uint16_t x0 = ldg16(xs, el), x1 = ldg16(xs, el + 64);
-                if (a.h_rot) {
-                    v0 = x0;
-                    v1 = x1;
-                } else {
-                    rotate_block(h2f(x0), h2f(x1), ldg16(suh, hb * 128 + el), ldg16(suh, hb * 128 + 64 + el), lane,
-                                 v0, v1);
-                    ep = et;
-                }
+            } else if (a.sorted[r] >= 0) {
+                gate_up_block<false>(a, a.cls[c], r, hb, jx, 1, lane, v0, v1);
             }
-            lds_put(A, q, kp, hb * 128, ep, v0, v1);
+            lds_put(A, q, kp, hb * 128, el, v0, v1);
         }
     }
     __syncthreads();
@@ -1975,12 +1963,13 @@ template <int NW> __device__ __forceinline__ void zero_dead_rows(const Exl3c4Lau
 }
 
 // The staged input of KS 64-k steps of a chunk of R = 16 NT rows: R rows x 4 KS groups of 16 halves, a group two 16-byte
-// loads, spread over 256 threads (H groups a thread; a slot past the last group reloads it,
-// so that the loads stay unconditional and their waits exact). Rows past the chunk load a copy of its last row. A
-// slot's address is the stage's base (wave-uniform: scalar registers) plus the slot's byte offset, fixed for the chunk
-// and held in a register (32 bits: 2 q pitch + 48 < 2^32 for the q < 96 rows of a chunk, which the host's choice of
-// the prefill path keeps), so the steps' loads take no address arithmetic. The groups land in LDS in row order, k in
-// order: pf_step pairs the decoded B registers to match.
+// loads, spread over 256 threads (H groups a thread; a slot past the last group reloads it, so that the loads stay
+// unconditional and their waits exact). Rows past the chunk load a copy of its last row. A slot's address is the stage's
+// base (wave-uniform: scalar registers) plus the slot's byte offset, fixed for the chunk and held in a register, so the
+// steps' loads take no address arithmetic. 32 bits hold it: row q <= 111 and group 4 KS - 1 <= 15 lie at most
+// 2 x (111 pitch + 240) bytes on, the group's end 32 more, below 2^32 up to the pitch of 2^24 halves that the host's
+// choice of the prefill path keeps. The groups land in LDS in row order, k in order: pf_step pairs the decoded B
+// registers to match.
 template <int NT, int KS> struct StageRegs {
     static constexpr int G = 64 * NT * KS;                        // groups a stage
     static constexpr int H = (G + 255) / 256;                     // slots a thread
