@@ -441,9 +441,10 @@ def extent_read_floor(torch, layers, draws, n):
 def measured_peaks(torch):
     """What this box reaches, on this library's own kernels (libexl3c4_calib.so, event-timed, best of 8): HBM read (a
     4 GiB stream, 16-byte loads, four in flight a thread), the VALU issue rate of the trellis decode's own
-    instructions (8 independent chains a wave, 4 to 8 waves a SIMD) and with it the engine clock under that load, and
-    the f16 MFMA rate (v_mfma_f32_16x16x32_f16, 8 independent chains a wave); beside them torch's plain copy and fill
-    and hipBLASLt's f16 GEMM (library work)."""
+    instructions (a mul1 pair: 2 v_bfe_u32, 2 v_mul_lo_u32, v_sad_u8, v_sad_hi_u8, v_pk_fma_f16; 8 independent chains
+    a wave, 4 to 8 waves a SIMD) and with it the engine clock under that load, and the f16 MFMA rate
+    (v_mfma_f32_16x16x32_f16, 8 independent chains a wave); beside them torch's plain copy and fill and hipBLASLt's
+    f16 GEMM (library work)."""
     C = calib()
     st = torch.cuda.current_stream().cuda_stream
     n = 1 << 30

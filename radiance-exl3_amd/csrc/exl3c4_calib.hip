@@ -67,12 +67,12 @@ __global__ __launch_bounds__(256) void k_read_runs(const uint64_t* __restrict__ 
     if (lane == 0 && acc == 0x9E3779B9u) out[0] = acc;             // almost never: keeps the reads live
 }
 
-// The VALU's issue rate on four-cycle instructions, in 8 independent chains a wave (not the latency): each round is the
-// mul1 pair by 16-bit products (2 v_pk_mul_lo_u16, 2 v_mad_u32_u16, v_sad_u8, v_sad_hi_u8, v_pk_fma_f16) on 8 sets,
-// 56 VALU instructions.
+// The decode's VALU instructions in 8 independent chains a wave (the issue rate, not the latency): each round is the mul1
+// pair as the kernels decode it (two states by v_bfe_u32, two v_mul_lo_u32, v_sad_u8, v_sad_hi_u8, v_pk_fma_f16) on 8
+// register sets, 56 VALU instructions, each a four-cycle one.
 __global__ __launch_bounds__(256) void k_valu(int rounds, uint32_t seed, uint32_t* out) {
     uint32_t r[8], y[8];
-    const uint32_t kh = 0x83DC0000u, cl = 0xD12Du, c64 = 0x64006400u, kinv = 0x1EEE1EEEu, kb = 0xC931C931u;
+    const uint32_t mul = 0x83DCD12Du, c64 = 0x64006400u, kinv = 0x1EEE1EEEu, kb = 0xC931C931u;
 #pragma unroll
     for (int q = 0; q < 8; ++q) r[q] = seed ^ (threadIdx.x * 0x9E3779B9u) ^ (q * 0x85EBCA6Bu);
     for (int it = 0; it < rounds; ++it) {
@@ -80,15 +80,15 @@ __global__ __launch_bounds__(256) void k_valu(int rounds, uint32_t seed, uint32_
         for (int q = 0; q < 8; ++q) {
             uint32_t ya, yb;
             asm volatile(
-                "v_pk_mul_lo_u16 %[ya], %[r], %[kh] op_sel:[0,0] op_sel_hi:[0,1]\n\t"
-                "v_pk_mul_lo_u16 %[yb], %[r], %[kh] op_sel:[1,0] op_sel_hi:[1,1]\n\t"
-                "v_mad_u32_u16 %[ya], %[r], %[cl], %[ya]\n\t"
-                "v_mad_u32_u16 %[yb], %[r], %[cl], %[yb] op_sel:[1,0,0,0]\n\t"
+                "v_bfe_u32 %[ya], %[r], 0, 16\n\t"
+                "v_bfe_u32 %[yb], %[r], 16, 16\n\t"
+                "v_mul_lo_u32 %[ya], %[ya], %[mul]\n\t"
+                "v_mul_lo_u32 %[yb], %[yb], %[mul]\n\t"
                 "v_sad_u8 %[ya], %[ya], 0, %[c64]\n\t"
                 "v_sad_hi_u8 %[ya], %[yb], 0, %[ya]\n\t"
                 "v_pk_fma_f16 %[r], %[ya], %[kinv], %[kb]"
                 : [ya] "=&v"(ya), [yb] "=&v"(yb), [r] "+v"(r[q])
-                : [kh] "s"(kh), [cl] "s"(cl), [c64] "s"(c64), [kinv] "s"(kinv), [kb] "v"(kb));
+                : [mul] "s"(mul), [c64] "s"(c64), [kinv] "s"(kinv), [kb] "v"(kb));
             y[q] = ya;
         }
     }
