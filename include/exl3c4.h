@@ -127,16 +127,16 @@ int64_t exl3c4_scratch_bytes_geom(int32_t op, int32_t n_class, const int32_t* ro
 int exl3c4_launch(const Exl3c4Op* op, void* scratch, int64_t scratch_bytes, void* stream);
 
 /* gate_up_down's single kernel (the decode path from EXL3C4_GD_FUSE_MIN_T sorted rows) orders its workgroups through
- * a block of counters -- a status word and two counters a sorted row (and a line a token for exl3c4_launch_gather) -- that must be zero when it starts and that it
- * leaves zero again when it ends well (each row's last down unit zeroes the row's). exl3c4_launch zeroes them in its
- * scratch before every launch (one more dispatch). exl3c4_launch_ctr takes them from `ctr` instead: a device block of
+ * a block of counters -- a status word and two counters a sorted row (and a line a token for exl3c4_launch_gather) --
+ * that must be zero when it starts and that it leaves zero again when it ends well (each row's last down unit zeroes
+ * the row's). exl3c4_launch zeroes them in its scratch before every launch (one more dispatch). exl3c4_launch_ctr takes them from `ctr` instead: a device block of
  * at least exl3c4_ctr_bytes, 256-B aligned, that the caller zeroed once (hipMemset) and keeps -- the reference's
  * counter pool, which its row instance's init allocates and zeroes and whose blocks the fused launch leaves zero
  * (kernels/exl3r4d/launch.c:311-324; the fused launch's `ctr` argument, launch.c:464-466). Given such a block, a decode
- * launch of at least four experts a token (top_k >= 4) runs as the single kernel below EXL3C4_GD_FUSE_MIN_T rows too,
- * with the same bits. The block's first int32 is
- * the status word exl3c4_scratch_status describes (0: good); after a launch that left it nonzero, zero the block again.
- * Two launches that may overlap (two streams) need two blocks; launches that share one are ordered on one stream. A
+ * launch of at least four experts a token (top_k >= 4) runs as the single kernel from 2 rows on, with the same bits (a
+ * block too small for its rows' counters, or misaligned, is not read below EXL3C4_GD_FUSE_MIN_T rows, and refused from
+ * there). The block's first int32 is the status word exl3c4_scratch_status describes (0: good); after a launch that
+ * left it nonzero, zero the block again. Two launches that may overlap (two streams) need two blocks; launches that share one are ordered on one stream. A
  * launch that does not run that kernel does not read ctr: exl3c4_launch_ctr is then exl3c4_launch. */
 int64_t exl3c4_ctr_bytes(const Exl3c4Op* op);
 int exl3c4_launch_ctr(const Exl3c4Op* op, void* scratch, int64_t scratch_bytes, void* stream, void* ctr,
@@ -169,16 +169,17 @@ int     exl3c4_launch_noalloc(const Exl3c4Op* op, void* stream);
 
 /* The kernels a launch can run: prep_gu's rotation; gate_up's GEMM (with its input rotation), then for gate_up alone
  * its epilogue; down's GEMM with its epilogue (in gate_up_down it also forms h from gate_up's partial sums); and
- * gate_up_down's single kernel, which runs both GEMMs in one dispatch at decode once T >= EXL3C4_GD_FUSE_MIN_T.
+ * gate_up_down's single kernel, which runs both GEMMs in one dispatch at decode: of a timed launch, which takes no
+ * counter block, from T >= EXL3C4_GD_FUSE_MIN_T.
  * exl3c4_launch_timed refuses (EXL3C4_E_INVAL) a kernel that the launch does not run. */
 enum { EXL3C4_K_PREP = 0, EXL3C4_K_GATE_UP = 1, EXL3C4_K_EPI_GU = 2, EXL3C4_K_DOWN = 3, EXL3C4_K_GATE_UP_DOWN = 4 };
 #define EXL3C4_GD_FUSE_MIN_T 32
 
 /* The least sorted-row count T at which gate_up, down and gate_up_down over n_expert experts take the prefill path (a
  * chunk plan and one GEMM kernel a projection, decoding each weight once a chunk of up to 112 rows of one expert, 96
- * where the launch's K exceed 4) rather than the decode kernels: max(64, ceil(7 n_expert / 8)) -- the crossover
- * measured on MI355X at the decode layer's experts. A function of T and n_expert only, never of the routing. A query
- * with no counterpart in the reference (whose rows split the band at M = 17, kernels/exl3r4d/rows.c:255-315). */
+ * where the launch's K exceed 4) rather than the decode kernels: max(64, ceil(7 n_expert / 8)), which lies between
+ * the crossovers measured on MI355X for even and for skewed routing. A function of T and n_expert only, never of the
+ * routing. A query with no counterpart in the reference (whose rows split the band at M = 17, kernels/exl3r4d/rows.c:255-315). */
 int64_t exl3c4_prefill_min_rows(int64_t n_expert);
 
 /* exl3c4_launch, with kernel `kernel` of the sequence dispatched so that the dispatch itself stamps ev_start and

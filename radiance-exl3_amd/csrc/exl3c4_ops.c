@@ -114,17 +114,18 @@ static int log2i(int v) {
 
 /* The prefill path (the rotation with the chunk plan, then one GEMM kernel a projection over chunks of up to 112 rows
  * of one expert) serves a launch of at least 64 sorted rows that average at least 7/8 of a row an expert: T >= 64 and
- * 8 T >= 7 n_expert (exl3c4_prefill_min_rows). Below it the decode kernels serve it (chunks of up to 16 rows, split-K;
- * gate_up_down as one kernel from EXL3C4_GD_FUSE_MIN_T rows). The rule lies where neither routing loses much (measured on
- * MI355X at the decode layer's experts, 512 experts, 2048 / 512, K = 4, top-10, the layer step in us by the decode
- * kernels / by the prefill kernels): softmax routing M = 32: 122 / 135, 40: 144 / 159, 48: 157 / 162, 56: 173 / 184,
- * 64: 187 / 185, 96: 238 / 211, 128: 269 / 235; a Zipf popularity 32: 97 / 103, 48: 135 / 110, 64: 173 / 132; hidden
- * 2560 32: 188 / 188, 40: 215 / 219, 64: 305 / 276; 128 experts top-8 24: 72 / 79, 32: 79 / 81, 48: 96 / 83. The
- * reference serves M >= 17 by its GEMM rows (kernels/exl3r4d/rows.c:255-315, kernels/exl3r4d/prefill.c:61-76); here the
- * decode kernels keep the band below the crossover. A function of
- * T, n_expert and the op's widths (never of the routing): the prefill GEMMs address a chunk's staged rows by 32-bit
- * byte offsets (2 x 111 x pitch + 64 < 2^32), so an input pitch past EXL3C4_PF_MAX_PITCH halves (the caller's x, the
- * rotated input's 2 x cols, h's rows / 2) keeps the decode kernels at any T. */
+ * 8 T >= 7 n_expert (exl3c4_prefill_min_rows). Below it the decode kernels serve it (chunks of up to four rows, 16 where
+ * a token has one expert; split-K; gate_up_down as one kernel from EXL3C4_GD_FUSE_MIN_T rows). The rule, one number for
+ * every routing, costs an evenly routed batch between it and that routing's own crossover up to 6% (45 to 60 tokens here),
+ * so that a skewed one there gains up to a fifth. Measured on MI355X at the decode layer's experts (512 experts,
+ * 2048 / 512, K = 4, top-10), the layer step in us by the decode kernels / by the prefill kernels: softmax routing
+ * M = 32: 122 / 135, 40: 144 / 159, 48: 157 / 162, 56: 173 / 184, 64: 187 / 185, 96: 238 / 211, 128: 269 / 235; a Zipf
+ * popularity 32: 97 / 103, 48: 135 / 110, 64: 173 / 132; hidden 2560 32: 188 / 188, 40: 215 / 219, 64: 305 / 276; 128
+ * experts top-8 24: 72 / 79, 32: 79 / 81, 48: 96 / 83. The reference serves M >= 17 by its GEMM rows
+ * (kernels/exl3r4d/rows.c:255-315, kernels/exl3r4d/prefill.c:61-76); here the decode kernels keep the band below. A
+ * function of T, n_expert and the op's widths (never of the routing): the prefill GEMMs address a chunk's staged rows by
+ * 32-bit byte offsets (2 x (111 pitch + 240) + 32 < 2^32), so an input pitch past EXL3C4_PF_MAX_PITCH halves (the
+ * caller's x, the rotated input's 2 x cols, h's rows / 2) keeps the decode kernels at any T. */
 #ifndef EXL3C4_PF_MIN_T
 #define EXL3C4_PF_MIN_T 64
 #endif
@@ -584,7 +585,7 @@ static int runs_kernel(const Exl3c4Op* o, const Carve* k, int kernel) {
  *   down          its GEMM, whose workgroups stage (and rotate) their rows and finish their output blocks
  *   gate_up_down  gate_up's GEMM, then down's, whose workgroups build h from gate_up's partial sums; from
  *                 GD_FUSE_MIN_T rows (or fewer, gd_few) both GEMMs in one kernel (launch_gd1)
- * Prefill (launch_prefill) plans 64-row chunks of one expert first and runs one GEMM kernel a projection. */
+ * Prefill (launch_prefill) plans chunks of one expert (up to 112 rows) first and runs one GEMM kernel a projection. */
 static int launch_impl(const Exl3c4Op* o, void* scratch, int64_t scratch_bytes, void* stream, const Ctx* t) {
     int rc;
     if (!o) return EXL3C4_E_INVAL;
