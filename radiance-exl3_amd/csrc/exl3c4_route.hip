@@ -223,12 +223,17 @@ __global__ __launch_bounds__(256) void k_router(const void* logits, int64_t n_to
 // What bounds it: a workgroup's chain -- three rounds of id loads, 40 LDS atomics a thread and two scans at 40,960
 // pairs -- so the time is nearly one workgroup's, however many run: 800 us in one workgroup of 8 waves before (its ranks
 // by readlane sweeps over every pair, twice), 14 us now, 401 -> 11 us at 20,480 pairs, 29 -> 6 at 1,280.
-constexpr int SC_THREADS = 1024, SC_SEG = 256, SC_LOADS = 16, SC_MAX_WG = 256;
+// LOADS: a thread's id loads in a round, no more than the pairs need (16 waves of which most load a copy of the last id
+// issue for longer than the few pairs take), as waves without a pair rank none. 1 / 80 / 320 / 1,280 pairs over 512
+// experts, us a launch of a chain of them: 4.76 / 4.90 / 4.87 / 5.28 with sixteen loads always, 2.50 / 3.69 / 4.31 / 4.69
+// now; the single workgroup before took 3.28 / 4.83 / 9.11 / 27.8.
+constexpr int SC_THREADS = 1024, SC_SEG = 256, SC_MAX_WG = 256;
 __device__ __forceinline__ int expert_of(int32_t id, int64_t base, int n_expert) {
     const int64_t g = (int64_t)id - base;
     return (g >= 0 && g < n_expert) ? (int)g : -1;
 }
 
+template <int LOADS>
 __global__ __launch_bounds__(SC_THREADS) void k_scatter(const int32_t* ids, uint32_t T, int64_t base, int32_t n_expert,
                                                         uint32_t seg, int32_t* sorted, int32_t* off, int32_t* count,
                                                         int32_t* row_of) {
@@ -241,15 +246,15 @@ __global__ __launch_bounds__(SC_THREADS) void k_scatter(const int32_t* ids, uint
     const int mine = tid < SC_SEG && lo + tid < hi ? ids[lo + tid] : 0;   // the first SC_SEG pairs, loaded ahead
     hist[tid] = hist[SC_THREADS + tid] = 0;
     __syncthreads();
-    for (uint32_t i0 = 0; i0 < T; i0 += SC_THREADS * SC_LOADS) {
-        int32_t f[SC_LOADS];
+    for (uint32_t i0 = 0; i0 < T; i0 += SC_THREADS * LOADS) {
+        int32_t f[LOADS];
 #pragma unroll
-        for (int j = 0; j < SC_LOADS; ++j) {
+        for (int j = 0; j < LOADS; ++j) {
             const uint32_t i = i0 + SC_THREADS * j + tid;
             f[j] = ids[i < T ? i : T - 1];
         }
 #pragma unroll
-        for (int j = 0; j < SC_LOADS; ++j) {
+        for (int j = 0; j < LOADS; ++j) {
             const uint32_t i = i0 + SC_THREADS * j + tid;
             const int e = i < T ? expert_of(f[j], base, n_expert) : -1;
             if (e >= 0) atomicAdd(&hist[(i < lo ? 0 : SC_THREADS) + e], 1);
@@ -281,12 +286,13 @@ __global__ __launch_bounds__(SC_THREADS) void k_scatter(const int32_t* ids, uint
         }
         __syncthreads();
         const int blk = wv & 3, part = wv >> 2;                   // SC_SEG / 64 of each
-        if (part <= blk) {
+        if (part <= blk && c0 + blk * 64 < hi) {                  // uniform in the wave, like the loop's end
             const int own = eid[blk * 64 + lane];
             const int upto = part < blk ? 64 : lane;
+            const int n = hi - c0 - part * 64 < 64 ? (int)(hi - c0) - part * 64 : 64;
             int r = 0;
 #pragma unroll 4
-            for (int j = 0; j < 64; j += 4) {
+            for (int j = 0; j < n; j += 4) {
                 const int4 q = *(const int4*)&eid[part * 64 + j];
                 r += (q.x == own && j < upto) + (q.y == own && j + 1 < upto) + (q.z == own && j + 2 < upto) +
                      (q.w == own && j + 3 < upto);
@@ -476,8 +482,9 @@ extern "C" int exl3c4_dev_scatter(const int32_t* ids, int64_t T, int64_t base, i
     const int64_t segs = T > 0 ? (T + SC_SEG - 1) / SC_SEG : 1;
     const int64_t per = row_of == ids ? segs : (segs + SC_MAX_WG - 1) / SC_MAX_WG;
     const unsigned wgs = (unsigned)((segs + per - 1) / per);
-    hipLaunchKernelGGL(k_scatter, dim3(wgs), dim3(SC_THREADS), 0, (hipStream_t)stream, ids, (uint32_t)T, base,
-                       n_expert, (uint32_t)(per * SC_SEG), sorted, off, count, row_of);
+    const auto f = T <= SC_THREADS ? k_scatter<1> : T <= 4 * SC_THREADS ? k_scatter<4> : k_scatter<16>;
+    hipLaunchKernelGGL(f, dim3(wgs), dim3(SC_THREADS), 0, (hipStream_t)stream, ids, (uint32_t)T, base, n_expert,
+                       (uint32_t)(per * SC_SEG), sorted, off, count, row_of);
     return launched();
 }
 

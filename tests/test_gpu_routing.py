@@ -110,6 +110,20 @@ def test_scatter_segments_match_the_oracle(torch_cuda, n_tok, top_k, n_expert, l
         assert np.array_equal(g, w_), name
 
 
+@pytest.mark.parametrize("T", [1, 2, 3, 63, 64, 65, 129, 193, 1023, 1024, 1025, 4095, 4096, 4097])
+def test_scatter_at_the_edges_of_its_loads_and_waves(torch_cuda, T):
+    """Pair counts around a wave's 64 and around what one, four and sixteen id loads a thread cover (1,024 and 4,096), with
+    dropped pairs, and with every pair on one expert."""
+    import oracle
+    torch = torch_cuda
+    rng = np.random.default_rng(T)
+    for n_expert, ids in ((1000, rng.integers(-1, 1001, (T, 1))), (5, np.full((T, 1), 3))):
+        ids = ids.astype(np.int32)
+        got, want = _scatter(torch, ids, n_expert), oracle.moe_scatter_full(ids, n_expert, 0)
+        for g, w_, name in zip(got, want, ("sorted_tok", "expert_offset", "expert_count", "row_of")):
+            assert np.array_equal(g, w_), name
+
+
 @pytest.mark.parametrize("n_tok,top_k,n_expert", [(8, 10, 512), (300, 1, 7), (2048, 10, 512), (4096, 10, 512)])
 def test_scatter_writes_row_of_over_the_ids(torch_cuda, n_tok, top_k, n_expert):
     """row_of the same buffer as expert_ids: each pair's row in the place of its expert, the other outputs as with a buffer
