@@ -26,8 +26,9 @@ extern "C" {
 #define EXL3C4_SYNC_DONE 32
 #define EXL3C4_SYNC_COUNT 16
 #define EXL3C4_SYNC_BLOCKS (64 - EXL3C4_SYNC_COUNT)
-/* polls (0.3 us or more each) after which a waiting down unit leaves its block where it may: a launch that runs alone
- * needed at most 44 (1 to 44 tokens, K 2..8, Zipf and even routing: waits of up to 20 us) */
+/* polls (0.3 us or more each) after which a down unit that waits for gate_up units leaves its block: at 512-wide experts a
+ * launch that runs alone needed at most 44 (1 to 44 tokens, K 2..8, Zipf and even routing), waits for h included; wider
+ * ones and long chunks may need more, at no measured cost (wait_gate_up) */
 #define EXL3C4_LEAVE_POLLS 128
 /* Rows of one chunk on the prefill path at most: seven MFMA row tiles share each decoded step where a launch's K are
  * at most 4, six (EXL3C4_PF_ROWS_WIDE) at larger K. */

@@ -806,10 +806,14 @@ __host__ __device__ __forceinline__ int gd_lists_log2(int64_t T, int nblk) {
 //              wait gives up all the same and sets the status word.)
 // one list     a gate_up unit of the row may still need a slot on another XCD, and the units of another launch that wait
 //              there may need the slot this unit holds (a cycle of two launches). So a unit that has polled
-//              a.leave_polls times leaves block b to the unit that forms h: it sets b's bit in the row's counter and
-//              ends, and the count of h, an addition to the same word, hands that unit every bit set before it. A unit
-//              whose bit came after the count finds h ready in the value it read and goes on. So each block is run once,
-//              and no unit holds its slot for another's start.
+//              a.leave_polls times while gate_up units of the row were missing leaves block b to the unit that forms h:
+//              it sets b's bit in the row's counter and ends, and the count of h, an addition to the same word, hands
+//              that unit every bit set before it. A unit whose bit came after the count finds h ready in the value it
+//              read and goes on. So each block is run once, and no unit holds its slot for another's start. Once the
+//              row's gate_up units have all counted, the unit that forms h runs and waits for nothing, and the others
+//              wait for it: the blocks of a row left to one unit run one after another, which a long chunk's slow h
+//              otherwise brought about in a launch alone (one expert's 40 rows at 4096 / 1536: 179 us by eight lists, 679
+//              with leaving by polls alone, 133 so; 40 rows at 4096 / 1024 119, 439, 96).
 // A status word already set when the wait begins gives up at once, before any counter is read: a block whose earlier
 // launch gave up may hold stale counts (a late gate_up count lands after the row's down units zeroed the row's
 // counters), so every later launch on it is void and reports it again -- in the same launch -- until the caller zeroes
@@ -829,7 +833,7 @@ __device__ __forceinline__ bool wait_gate_up(const Exl3c4Launch& a, int i, int b
         bool give_up = (st & 1) != 0;
         int left = 0;
         for (int n = 1; !give_up && count_of(c) < want; ++n) {
-            if (leaves && n > a.leave_polls) {
+            if (leaves && n > a.leave_polls && count_of(c) < want - 1) {
                 c = __hip_atomic_fetch_or(cnt, 1ull << (EXL3C4_SYNC_COUNT + b), __ATOMIC_RELAXED,
                                           __HIP_MEMORY_SCOPE_AGENT);
                 left = count_of(c) < want;

@@ -5,7 +5,8 @@ The kernel's rules, as the model states them. Units are numbered gate_up first (
 dealt to the XCDs in turn: unit g to XCD g mod X (one list), or row i's all to XCD i mod X (a list an XCD). A gate_up unit
 waits for nothing: it adds one to its row's word; the unit whose addition is the row's last forms h and adds one more,
 and runs the blocks that the word it read names as left. A down unit polls its row's word for that last count. In one list
-it may give its slot back instead: it sets its block's bit in the word and leaves, unless the value it read shows h ready.
+it may give its slot back instead while the row's gate_up units are not all counted (once they are, the unit that forms h
+runs and waits for nothing): it sets its block's bit in the word and leaves, unless the value it read shows h ready.
 Each block's unit then counts; the row's last one clears the word.
 
 What holds in every order: every launch ends (no state without a next step but the end), each block is run once, and
@@ -97,7 +98,9 @@ class Model:
         elif pc == DN:
             if cnt >= want:
                 yield self._set(s, run=self._add(run, (la, x, i, RUN, u, 0)))
-            if self.leaves:              # the polls are spent, whatever the last one read
+            # the polls are spent: the unit leaves while gate_up units of the row are missing in the value it read last --
+            # which may be an older one than the word now ("late"), or not ("early")
+            if self.leaves == "late" or (self.leaves == "early" and cnt < self.ugu):
                 t = self._set(s, words=self._word(s[2], la, i, (cnt, left | 1 << u, done)))
                 yield self._set(t, run=self._add(run, (la, x, i, RUN, u, 0)) if cnt >= want else run)
         else:
@@ -130,14 +133,14 @@ def _holds(m):
         assert all(w == (0, 0, 0) for w in s[2]) and all(n == 1 for n in s[3])
 
 
-@pytest.mark.parametrize("one_list", [True, False])
+@pytest.mark.parametrize("one_list,leaves", [(True, "late"), (True, "early"), (False, "")])
 @pytest.mark.parametrize("launches,rows,ugu,nblk,slots", [(2, 2, 1, 2, 1), (2, 2, 2, 2, 1), (2, 3, 1, 1, 2), (1, 2, 2, 3, 3)])
-def test_every_order_of_starts_ends_with_each_block_run_once(one_list, launches, rows, ugu, nblk, slots):
-    _holds(Model(2, slots, launches, rows, ugu, nblk, one_list, leaves=one_list))
+def test_every_order_of_starts_ends_with_each_block_run_once(one_list, leaves, launches, rows, ugu, nblk, slots):
+    _holds(Model(2, slots, launches, rows, ugu, nblk, one_list, leaves))
 
 
 def test_a_wait_that_holds_its_slot_across_the_xcds_does_not_end():
     """The rule that the model is there to refuse: one list, and a down unit that only waits."""
-    stuck, _ = walk(Model(2, 1, 2, 2, 1, 2, one_list=True, leaves=False))
+    stuck, _ = walk(Model(2, 1, 2, 2, 1, 2, one_list=True, leaves=""))
     assert stuck
-    _holds(Model(2, 1, 1, 2, 1, 2, one_list=True, leaves=False))    # a launch alone ends
+    _holds(Model(2, 1, 1, 2, 1, 2, one_list=True, leaves=""))    # a launch alone ends

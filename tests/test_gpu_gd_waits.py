@@ -24,7 +24,8 @@ def torch_cuda():
     (7, 8, 20, [(256, 384)], 8, 8, "mcg", 0.1),                 # chunks of several rows
     (1, 41, 64, [(6144, 128)], 2, 2, "mul1", 0.0),              # 48 blocks: the most a row's counter has a bit for
     (1, 41, 64, [(6272, 128)], 2, 2, "3inst", 0.0),             # 49: a list an XCD, no unit leaves
-    (3, 13, 48, [(512, 256)], 5, 5, "mul1", 0.0)])              # 39 rows: a list an XCD
+    (3, 13, 48, [(512, 256)], 5, 5, "mul1", 0.0),               # 39 rows: a list an XCD
+    (56, 1, 3, [(256, 1536)], 4, 4, "mul1", 0.0)])              # chunks of 16 rows, an h of twelve blocks: slow to form
 def test_units_that_leave_give_the_bits_of_units_that_wait(torch_cuda, n_tok, top_k, n_expert, geoms, bits, dn_bits, cb,
                                                            drop):
     import exl3c4 as ex
