@@ -68,19 +68,21 @@ static int64_t chunk_bound(int64_t T, int64_t n_expert, int ch) {
 #endif
 
 /* gate_up's split-K on the decode path, from T, M and the geometry (never the routing): the most splits -- a power of
- * two, at most 16 and at most one a 128-block of k -- that keep the launch's gate_up units (chunks x n_grp x S) at
- * most GU_UNITS. A split shortens a unit's chain of code loads (and so the wait of the row's down units for its last
- * gate_up unit) and adds a unit's fixed start-up; on configs[2] (80 chunks x 8 groups) S = 4, 2560 units against
- * about 1790 resident workgroups, measured 1.7 us a layer step faster than S = 2 (every unit resident at once) and
- * 5 us faster than S = 8. Then more splits while a split's staged rows would take more LDS than GU_LDS_BUDGET (which
- * keeps 7 workgroups a CU). The limit, 4096 / 5000 / 6500 / 8200 units, the layer step in us: 8 tokens 47.2 / 47.2 / 51.6 /
- * 51.6, 12 tokens 61.1 / 62.1 / 61.7 / 62.1, 16 tokens 76.4 / 75.5 / 76.7 / 77.3, 32 tokens 119.0 / 119.7 / 122.0 / 123.6,
- * 16 tokens of width 256 33.3 / 33.5 / 38.7 / 38.4; the ops one by one 12 tokens 70.7 / 67.1 / 67.0 / 67.1, 14 tokens of
- * widths 384 and 256 74.0 / 68.3 / 68.1 / 68.2, 14 tokens of top-6 over 128 experts of width 768 (5,088 units) 68.9 / 69.2 /
- * 64.9 / 64.8, 8 tokens 51.9 / 51.9 / 53.6 / 53.5. One rule for gate_up and gate_up_down: the same splits, so that
- * gate_up_down gives its pair's bits. */
+ * two, at most 16 and at most one a 128-block of k -- that keep chunk_bound x n_grp x S at most GU_UNITS. (chunk_bound is
+ * the most chunks any routing makes: an even one has fewer, 8 tokens of top-10 about 76 of 101.) A split shortens a
+ * unit's chain of code loads (and so the wait of the row's down units for its last gate_up unit) and adds a unit's fixed
+ * start-up. Then more splits while a split's staged rows would take more LDS than GU_LDS_BUDGET (which keeps 7 workgroups
+ * a CU).
+ * The limit serves gate_up_down, the layer's own launch: at 4096 / 5120 / 6400, the layer step in us where they differ
+ * (2048 / 512, 512 experts, top-10 unless said): 6 tokens 39.6 / 41.4 / 41.7, 12 tokens 59.5 / 60.6 / 60.1, 24 tokens 99.7 /
+ * 101.6 / 101.8, 2560 / 640 at 10 tokens 74.3 / 77.5 / 76.9, width 768 at 8 tokens 61.4 / 62.9 / 63.4, 2560 / 384 top-8 at 20
+ * tokens 74.5 / 76.7 / 76.3, 7 tokens 41.4 / 41.6 / 44.7, 26 tokens 106.0 / 107.7 / 109.8; width 768 of top-6 over 128 experts
+ * at 14 tokens alone is faster with more, 61.9 / 59.4 / 59.8. It costs the ops launched one by one, whose gate_up has no
+ * other units to run beside: 12 tokens 70.9 / 67.8 / 67.1, 2560 / 640 at 10 tokens 85.9 / 84.0 / 83.9, 2560 / 384 at 20
+ * tokens 85.1 / 82.2 / 82.1, width 768 at 14 tokens 67.0 / 63.3 / 64.0, 6 tokens 44.0 / 44.4 / 44.3. One rule for both: the
+ * same splits, so that gate_up_down gives its pair's bits. */
 #ifndef GU_UNITS
-#define GU_UNITS 5120
+#define GU_UNITS 4096
 #endif
 #ifndef GU_LDS_BUDGET
 #define GU_LDS_BUDGET (20 * 1024)

@@ -154,3 +154,19 @@ def test_launch_gather_refuses_like_launch_and_moe_gather():
     o = _op(op=exl3c4.GU_DN, M=8, top_k=10, E=64)
     assert exl3c4.ctr_bytes(o) >= (80 + 1 + 8) * 256          # a counter line a row and a token
 
+
+
+@pytest.mark.parametrize("M,top_k,E,H,W,splits", [
+    (8, 10, 512, 2048, 512, 4), (12, 10, 512, 2048, 512, 2), (24, 10, 512, 2048, 512, 1), (10, 10, 512, 2560, 640, 2),
+    (14, 6, 128, 2048, 768, 2), (4, 10, 512, 2560, 640, 4), (4, 10, 512, 1536, 384, 4)])
+def test_gate_ups_splits_keep_the_launch_within_its_units(M, top_k, E, H, W, splits):
+    """At most 4,096 units (the most chunks a routing makes x groups of strips x splits) from 32 rows, no split count that
+    idles more than an eighth of k's blocks, and gate_up_down's the same as gate_up's."""
+    for op in (exl3c4.GATE_UP, exl3c4.GU_DN):
+        o = _op(op=op, M=M, top_k=top_k, E=E, H=H, W=W)
+        off, pitch, stride, n = C.c_int64(), C.c_int64(), C.c_int64(), C.c_int32()
+        assert exl3c4.lib().exl3c4_scratch_partials(C.byref(o), 0, C.byref(off), C.byref(pitch), C.byref(stride),
+                                                    C.byref(n)) == 0
+        assert n.value == splits
+    T = M * top_k
+    assert (T // 4 + min(E, T) + 1) * (2 * W // 128) * splits <= 4096
