@@ -133,8 +133,8 @@ int exl3c4_launch(const Exl3c4Op* op, void* scratch, int64_t scratch_bytes, void
  * at least exl3c4_ctr_bytes, 256-B aligned, that the caller zeroed once (hipMemset) and keeps -- the reference's
  * counter pool, which its row instance's init allocates and zeroes and whose blocks the fused launch leaves zero
  * (kernels/exl3r4d/launch.c:311-324; the fused launch's `ctr` argument, launch.c:464-466). Given such a block, a decode
- * launch of at least four experts a token (top_k >= 4) runs as the single kernel from 2 rows on, with the same bits (a
- * block too small for its rows' counters, or misaligned, is not read below EXL3C4_GD_FUSE_MIN_T rows, and refused from
+ * launch of at least four experts a token (top_k >= 4) of width at most 768 (gate_up's rows / 2) runs as the single kernel
+ * from 2 rows on, with the same bits (a block too small for its rows' counters, or misaligned, is not read below EXL3C4_GD_FUSE_MIN_T rows, and refused from
  * there). The block's first int32 is the status word exl3c4_scratch_status describes (0: good); after a launch that
  * left it nonzero, zero the block again. Two launches that may overlap (two streams) need two blocks; launches that share one are ordered on one stream. A
  * launch that does not run that kernel does not read ctr: exl3c4_launch_ctr is then exl3c4_launch. */
@@ -205,7 +205,7 @@ int exl3c4_scratch_partials(const Exl3c4Op* op, int32_t gemm, int64_t* offset, i
                             int32_t* splits);
 
 /* exl3c4_launch_gather, whose single kernel's waiting down units leave their blocks to the unit that forms the row's h
- * after `polls` polls (0 .. 128; a launch's own number is 128, more than one that runs alone needs): the same bits,
+ * after `polls` polls that found gate_up units missing (0 .. 128; a launch's own number is 128): the same bits,
  * by the path that a launch takes beside others. EXL3C4_E_INVAL for another `polls`. A checker's entry; no counterpart in
  * the reference. */
 int exl3c4_launch_leaving(const Exl3c4Op* op, void* scratch, int64_t scratch_bytes, void* stream, void* ctr,

@@ -67,6 +67,23 @@ static int64_t chunk_bound(int64_t T, int64_t n_expert, int ch) {
 #define GD_FUSE_ROWS EXL3C4_GD_FUSE_MIN_T
 #endif
 
+/* With a counter block from the caller (exl3c4_launch_ctr, exl3c4_launch_gather), also below GD_FUSE_ROWS where a token
+ * has at least GD_FEW_TOP_K experts: they are distinct, so at least that many chunks of at most M rows are live and the
+ * kernel's chain a row runs over several of them at once (a single expert's 16 rows, measured, took 66 us there against
+ * 31 as three kernels). Without a block the counters' fill would be a dispatch of its own, and the three kernels stay. The
+ * step in us as three kernels / as one (512 experts, top-10, K = 4, the gather inside): 1 token 31.2 / 26.1, 2 tokens
+ * 35.0 / 29.3, 3 tokens 37.7 / 31.6; top-4 of 16 experts, 7 tokens 30.7 / 29.7; top-2 of 8 experts, 8 tokens 28.0 /
+ * 29.2 (so not below four). And where h has at most GD_FEW_BLOCKS 128-blocks: one workgroup forms a chunk's h, its
+ * blocks four at a time, and each down unit stages them so, where the three kernels spread them over the chip. Three
+ * kernels / one: width 768 top-8 of 128 at 3 tokens 41.9 / 38.2, top-4 at 7 tokens 43.2 / 38.3; width 1024 top-4 of 64 at 3, 5
+ * and 7 tokens 40.9 / 42.0, 49.6 / 51.5, 59.8 / 60.8; 4096 / 1536 top-4 of 16 at 1, 4 and 7 tokens 40.2 / 45.1, 63.2 / 68.3,
+ * 82.4 / 96.2; 2048 / 1408 top-6 of 64 at 2 and 5 tokens 42.7 / 41.1, 59.8 / 61.9. */
+#define GD_FEW_TOP_K 4
+#define GD_FEW_BLOCKS 6
+static int few_one(const Exl3c4Op* o, int64_t gu_rows) {
+    return o->top_k >= GD_FEW_TOP_K && gu_rows / 256 <= GD_FEW_BLOCKS;
+}
+
 /* gate_up's split-K on the decode path, from T, M and the geometry (never the routing): the most splits -- a power of
  * two, at most 16 and at most one a 128-block of k -- that keep chunk_bound x n_grp x S at most GU_UNITS. (chunk_bound is
  * the most chunks any routing makes: an even one has fewer, 8 tokens of top-10 about 76 of 101.) A split shortens a
@@ -91,19 +108,30 @@ static int64_t chunk_bound(int64_t T, int64_t n_expert, int ch) {
  * resident at once either way, and a split more only adds its start-up, its stores and its count. Measured (512 experts,
  * 2048 / 512, K = 4, the whole step in us, limits 4096 / 2100 / 1400 / 700 with gate_up_down as one kernel): 1 token
  * 28.3 / 26.9 / 26.7 / 25.6, 2 tokens 32.3 / 28.9 / 29.3 / 29.4, hidden 2560 and 1 token 36.2 / 32.0 / 31.7 / 33.5; as
- * three kernels, 4096 / 1400: 2 tokens 37.9 / 35.0, 8 tokens of top-2 over 8 experts 29.7 / 28.0. One expert a token
- * (top_k 1) may mean one live expert, whose few units need the splits: it keeps GU_UNITS. */
+ * three kernels, 4096 / 1400: 2 tokens 37.9 / 35.0, 8 tokens of top-2 over 8 experts 29.7 / 28.0. But a unit that still has
+ * more than FEW_BLOCKS 128-blocks of k (FEW_BLOCKS_ONE where the launch may be one kernel) is split on, up to GU_UNITS: wide
+ * experts reach the limit with units of 16 blocks and more, whose chain of loads is then the launch. Limits of 1024 alone /
+ * on beyond 8 blocks / beyond 4, the layer step: 4096 / 1536 top-2 of 8 at 4, 8 and 15 tokens 48.5 / 44.4 / 42.2, 62.2 / 54.8 /
+ * 53.0, 76.3 / 65.0 / 62.6, 2048 / 1408 top-6 of 64 at 3 tokens as three kernels 52.0 (8) / 48.7 (4); as one kernel 2048 / 512
+ * top-10 of 512 at 3 tokens 31.4 / 31.2 / 32.4, 2560 / 640 42.0 / 41.9 / 44.5, 7168 / 256 top-8 of 256 at 2 tokens 32.7 / 32.7 /
+ * 36.2. One expert a token (top_k 1) may mean one live expert, whose few units need the splits: it keeps GU_UNITS. */
 #define GU_UNITS_FEW 1024
+#define FEW_BLOCKS 4
+#define FEW_BLOCKS_ONE 8
 /* Whether s splits share nb 128-blocks of k without idling more than an eighth of them: a unit takes ceil(nb / s)
  * blocks, so 20 blocks in 8 splits run as long as 24 (the last split has none) and 12 in 8 as long as 16. Only where the
  * units are many: the few of GU_UNITS_FEW and of one expert a token gain from the shorter unit all the same. The step
  * without / with the rule, us, 4 tokens: 2560 / 640 49.7 / 47.9, op by op 51.0 / 49.1; 1536 / 384 31.0 / 28.0. */
 static int even_split(int64_t nb, int s) { return 8 * ((nb + s - 1) / s * s - nb) <= nb; }
-static int ksplit_for(int64_t T, int64_t top_k, int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max, int ch) {
-    const int64_t units = T < GD_FUSE_ROWS && top_k >= 2 ? GU_UNITS_FEW : GU_UNITS;
-    const int many = T >= GD_FUSE_ROWS && top_k >= 2;
+static int ksplit_for(int64_t T, int64_t top_k, int64_t chunks, int64_t n_grp, int64_t nb_min, int64_t nb_max, int ch,
+                      int one) {
+    const int few = T < GD_FUSE_ROWS && top_k >= 2;
+    const int64_t blocks = one ? FEW_BLOCKS_ONE : FEW_BLOCKS;
     int s = 1;
-    while (s < 16 && 2 * s <= nb_min && chunks * n_grp * 2 * s <= units && (!many || even_split(nb_max, 2 * s))) s *= 2;
+    while (s < 16 && 2 * s <= nb_min && chunks * n_grp * 2 * s <= GU_UNITS &&
+           (few ? chunks * n_grp * 2 * s <= GU_UNITS_FEW || (nb_max + s - 1) / s > blocks
+                : top_k < 2 || even_split(nb_max, 2 * s)))
+        s *= 2;
     while (s < 16 && 2 * s <= nb_max && (int64_t)ch * (((nb_max + s - 1) / s) * 128 + 8) * 2 > GU_LDS_BUDGET) s *= 2;
     return s;
 }
@@ -141,15 +169,6 @@ static int prefill_path(const Exl3c4Op* o, int64_t T) {
     return o->op != EXL3C4_PREP_GU && T >= exl3c4_prefill_min_rows(o->n_expert) && pitch <= EXL3C4_PF_MAX_PITCH &&
            max_rows(o) / 2 <= EXL3C4_PF_MAX_PITCH;
 }
-
-/* With a counter block from the caller (exl3c4_launch_ctr, exl3c4_launch_gather), also below GD_FUSE_ROWS where a token
- * has at least GD_FEW_TOP_K experts: they are distinct, so at least that many chunks of at most M rows are live and the
- * kernel's chain a row runs over several of them at once (a single expert's 16 rows, measured, took 66 us there against
- * 31 as three kernels). Without a block the counters' fill would be a dispatch of its own, and the three kernels stay. The
- * step in us as three kernels / as one (512 experts, top-10, K = 4, the gather inside): 1 token 31.2 / 26.1, 2 tokens
- * 35.0 / 29.3, 3 tokens 37.7 / 31.6; top-4 of 16 experts, 7 tokens 30.7 / 29.7; top-2 of 8 experts, 8 tokens 28.0 /
- * 29.2 (so not below four). */
-#define GD_FEW_TOP_K 4
 
 /* Below that, from GEPI_ROWS rows, gate_up_down forms h once a (row, 128-block) with gate_up's epilogue kernel (a wave
  * each, all in parallel) and down stages it as given; with fewer, down's workgroups form their chunk's h while staging
@@ -211,7 +230,8 @@ static void carve(const Exl3c4Op* o, int64_t T, Carve* k) {
         }
         int s = 1;
         if (!k->pf) {   /* split-K from T, M and the geometry: ksplit_for */
-            s = ksplit_for(T, o->top_k, chunk_bound(T, o->n_expert, k->chunk), rc / 128, nb_min, nb_max, k->chunk);
+            s = ksplit_for(T, o->top_k, chunk_bound(T, o->n_expert, k->chunk), rc / 128, nb_min, nb_max, k->chunk,
+                           few_one(o, rc));
             k->gu_lds_pitch = (int)(((nb_max + s - 1) / s) * 128 + 8);
         }
         k->split_gu = s;
@@ -558,7 +578,7 @@ static int launch_gd1(const Exl3c4Op* o, const Carve* k, char* s, void* stream, 
 /* Whether a launch given the counter block `ctr` runs gate_up_down's single kernel below GD_FUSE_ROWS rows: a block too
  * small for it (need bytes) leaves the launch as it is without one. */
 static int gd_few(const Exl3c4Op* o, const Carve* k, const void* ctr, int64_t ctr_bytes, int64_t need) {
-    return k->h_gepi && gd_pair(o) && o->T > 0 && o->top_k >= GD_FEW_TOP_K && ctr && ctr_bytes >= need &&
+    return k->h_gepi && gd_pair(o) && o->T > 0 && few_one(o, max_rows(o)) && ctr && ctr_bytes >= need &&
            (uintptr_t)ctr % 256 == 0;
 }
 

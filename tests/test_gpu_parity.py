@@ -466,16 +466,18 @@ def test_few_rows_with_a_counter_block_run_as_one_kernel(torch_cuda, n_tok, top_
         assert bool((ctr.view == (0x5A if small else 0)).all()) and ctr.ok()
 
 
-@pytest.mark.parametrize("n_tok,top_k,lines,reads", [
-    (2, 8, 0, False),                                           # no block: three kernels, then the gather's own
-    (5, 3, 64, False),                                          # fewer than four experts a token: as without a block
-    (15, 2, 64, False),
-    (2, 8, 16, False),                                          # a line short of the status word and the rows' counters
-    (2, 8, 17, True),                                           # the rows' alone: one kernel, then the gather's own
-    (3, 10, 33, True),                                          # a line short of the gather's
-    (3, 10, 34, True),                                          # all of them: the gather in the kernel
+@pytest.mark.parametrize("n_tok,top_k,lines,reads,width", [
+    (2, 8, 0, False, 256),                                      # no block: three kernels, then the gather's own
+    (5, 3, 64, False, 256),                                     # fewer than four experts a token: as without a block
+    (15, 2, 64, False, 256),
+    (2, 8, 16, False, 256),                                     # a line short of the status word and the rows' counters
+    (2, 8, 17, True, 256),                                      # the rows' alone: one kernel, then the gather's own
+    (3, 10, 33, True, 256),                                     # a line short of the gather's
+    (3, 10, 34, True, 256),                                     # all of them: the gather in the kernel
+    (2, 8, 64, True, 768),                                      # the widest h that the kernel takes below 32 rows
+    (2, 8, 64, False, 896),
 ])
-def test_launch_gather_below_32_rows_by_its_counter_block(torch_cuda, n_tok, top_k, lines, reads):
+def test_launch_gather_below_32_rows_by_its_counter_block(torch_cuda, n_tok, top_k, lines, reads, width):
     """exl3c4_launch_gather of 15 to 30 rows, with a counter block of `lines` lines of 256 bytes: y and out bit for bit
     those of exl3c4_launch and exl3c4_moe_gather; a block that the launch is not to read (its bytes anything) stays as it
     was, one that it reads (zero) is left zero."""
@@ -483,7 +485,7 @@ def test_launch_gather_below_32_rows_by_its_counter_block(torch_cuda, n_tok, top
     import oracle
     torch = torch_cuda
     n_expert = 12 if top_k <= 8 else 16
-    case = Case(seed=620 + 10 * n_tok + top_k, n_tok=n_tok, top_k=top_k, n_expert=n_expert, geoms=[(512, 256)], bits=4,
+    case = Case(seed=620 + 10 * n_tok + top_k, n_tok=n_tok, top_k=top_k, n_expert=n_expert, geoms=[(512, width)], bits=4,
                 cb="mul1")
     dev = Dev(case)
     assert 2 <= case.T < ex.GD_FUSE_MIN_T

@@ -170,3 +170,17 @@ def test_gate_ups_splits_keep_the_launch_within_its_units(M, top_k, E, H, W, spl
         assert n.value == splits
     T = M * top_k
     assert (T // 4 + min(E, T) + 1) * (2 * W // 128) * splits <= 4096
+
+
+@pytest.mark.parametrize("M,top_k,E,H,W,splits", [
+    (1, 10, 512, 2048, 512, 4), (3, 10, 512, 2560, 640, 4), (2, 8, 256, 7168, 256, 8),       # eight blocks a unit, or 1,024 units
+    (4, 2, 8, 4096, 1536, 8), (15, 2, 8, 4096, 1536, 8), (3, 6, 64, 2048, 1408, 4),          # four blocks, or 4,096
+    (8, 2, 8, 2048, 512, 8), (16, 1, 64, 4096, 1536, 8)])
+def test_gate_ups_splits_below_32_rows(M, top_k, E, H, W, splits):
+    """At most 1,024 units, and beyond them up to 4,096 while a unit holds more 128-blocks of k than it may: eight where the
+    launch may be gate_up_down's single kernel (four experts a token, six blocks of h), four otherwise. The same for both."""
+    for op in (exl3c4.GATE_UP, exl3c4.GU_DN):
+        off, pitch, stride, n = C.c_int64(), C.c_int64(), C.c_int64(), C.c_int32()
+        assert exl3c4.lib().exl3c4_scratch_partials(C.byref(_op(op=op, M=M, top_k=top_k, E=E, H=H, W=W)), 0, C.byref(off),
+                                                    C.byref(pitch), C.byref(stride), C.byref(n)) == 0
+        assert n.value == splits
