@@ -118,6 +118,18 @@ static int few_one(const Exl3c4Op* o, int64_t gu_rows) {
 #define GU_UNITS_FEW 1024
 #define FEW_BLOCKS 4
 #define FEW_BLOCKS_ONE 8
+/* An op launched alone (gate_up or down) takes its chunks larger than gate_up_down's where an expert has more than two
+ * rows by the batch's average: no row's h waits on a chunk there, so a longer run is best decoded once. The splits stay
+ * gate_up_down's (the same bits), and gate_up's staged rows at most 2 GU_LDS_BUDGET. Chunks of 4 / of up to 16, prep, gate_up
+ * and down in us: 4096 / 1536 top-2 of 8, 16 tokens 55.0 / 55.0, 20 64.1 / 58.7, 31 87.9 / 64.6, top-4 of 16 at 12 and 15 tokens
+ * 84.5 / 75.3, 93.5 / 79.2, 2048 / 768 top-2 of 4 at 24 tokens 38.4 / 31.6, 2048 / 512 top-4 of 16 at 15 tokens 37.3 / 34.2.
+ * gate_up_down itself is the faster with four: top-2 of 8, 31 tokens, 48.0 / 63.6 (2048 / 512). */
+static int chunk_alone(const Exl3c4Op* o, int64_t T, int ch, int lds_pitch) {
+    if (o->op == EXL3C4_GU_DN || o->top_k < 2 || T <= 2 * o->n_expert) return ch;
+    while (ch < EXL3C4_CHUNK_ROWS && ch < o->M && (int64_t)2 * ch * lds_pitch * 2 <= 2 * GU_LDS_BUDGET) ch <<= 1;
+    return ch;
+}
+
 /* Whether s splits share nb 128-blocks of k without idling more than an eighth of them: a unit takes ceil(nb / s)
  * blocks, so 20 blocks in 8 splits run as long as 24 (the last split has none) and 12 in 8 as long as 16. Only where the
  * units are many: the few of GU_UNITS_FEW and of one expert a token gain from the shorter unit all the same. The step
@@ -234,6 +246,7 @@ static void carve(const Exl3c4Op* o, int64_t T, Carve* k) {
                            few_one(o, rc));
             k->gu_lds_pitch = (int)(((nb_max + s - 1) / s) * 128 + 8);
         }
+        if (!k->pf) k->chunk = chunk_alone(o, T, k->chunk, k->gu_lds_pitch);
         k->split_gu = s;
         k->part_pitch = rc;
         off += ALIGN_UP(s * T * rc * 4, 256);
@@ -247,6 +260,7 @@ static void carve(const Exl3c4Op* o, int64_t T, Carve* k) {
     }
     k->dacc = off;
     if (dn) {
+        if (!gu && !k->pf) k->chunk = chunk_alone(o, T, k->chunk, 0);
         /* down's geometry: its own classes, or gate_up_down's [cols, rows / 2] */
         int64_t nmax = 0, kmax = 0;
         for (int c = 0; c < o->n_class; ++c) {
