@@ -392,7 +392,7 @@ class Dev:
                                dn_bits=0 if c.dn_bits == c.bits else c.dn_bits)
 
     def gate_up_down(self):
-        """gate_up_down's output; self.status is then None (two kernels) or 0 (one kernel, which went well)."""
+        """gate_up_down's output; self.status is then None (separate kernels) or 0 (one kernel, which went well)."""
         N = max(d["rows"] for d in self.tabs["dn"])
         y = self.out(N)
         self._run(self.gd_op(y), y)

@@ -10,7 +10,7 @@
               y bf16) a one-ulp flip of h, which a different summation order alone causes, is spread by down, and the
               layer output measures max-abs 9.1e-3 x RMS (rel-L2 3.3e-4).
   configs[3]  the prefill layer: 2048 tokens, Zipf(1.1) top-10 over the same 512 experts (20,480 rows, hot experts
-              of many 64-row chunks), against the oracle's gate_up_down; gate_up_down == its pair, zero rows, replay,
+              of many chunks), against the oracle's gate_up_down; gate_up_down == its pair, zero rows, replay,
               the checked f32 sums of sampled rows (the hottest expert's among them) within 2e-3 x RMS. And a smaller
               prefill (256 tokens over 32 experts) through every op against the oracle.
   configs[4]  one decode layer at each K in {2, 3, 6, 8} against the oracle, and the mixed-K layer (gate_up at K_g,
@@ -199,7 +199,7 @@ def test_middle_band_against_the_oracle(layer, M):
 
 def test_prefill_multichunk_hot_experts_through_every_op(torch_cuda):
     """The prefill path at the layer's shapes against the oracle op by op: 256 tokens, Zipf top-10 over 32 experts
-    (2560 rows, the hottest of several 64-row chunks)."""
+    (2560 rows, the hottest of several chunks)."""
     import exl3c4
     case = Case(seed=20261017, n_tok=256, top_k=10, n_expert=32, geoms=[(2048, 512)], bits=4, cb="mul1",
                 routing="zipf", drop=0.01, protect_tail=3)
